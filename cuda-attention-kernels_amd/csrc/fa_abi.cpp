@@ -115,6 +115,35 @@ fa_status fa_attention_fwd(const fa_fwd_params* p, void* stream) {
   return FA_OK;
 }
 
+size_t fa_attention_fwd_workspace_bytes(const fa_fwd_params* p) {
+  if (validate(p, /*varlen=*/false, /*fp8_ok=*/false, /*generic_ok=*/true) != FA_OK) return 0;
+  if (p->batch == 0 || p->seqlen_q == 0) return 0;
+  return fa::fwd_workspace_bytes(*p);
+}
+
+fa_status fa_attention_fwd_ws(const fa_fwd_params* p, void* workspace, size_t workspace_bytes, void* stream) {
+  g_last_error.clear();
+  fa_status st = validate(p, /*varlen=*/false, /*fp8_ok=*/false, /*generic_ok=*/true);
+  if (st != FA_OK) return st;
+  if (p->lse != nullptr && (p->lse_stride_b < 0 || p->lse_stride_h < 0))
+    return fail(FA_ERR_INVALID_ARGUMENT, "negative LSE stride");
+  if (p->batch == 0 || p->seqlen_q == 0) return FA_OK;
+  const size_t need = fa::fwd_workspace_bytes(*p);
+  if (need > 0) {
+    if (workspace == nullptr || workspace_bytes < need) {
+      char buf[160];
+      snprintf(buf, sizeof(buf), "prefill workspace too small: need %zu bytes, got %zu", need,
+               workspace == nullptr ? (size_t)0 : workspace_bytes);
+      return fail(FA_ERR_WORKSPACE, buf);
+    }
+    if (!aligned(workspace, 16)) return fail(FA_ERR_WORKSPACE, "workspace must be 16-byte aligned");
+  }
+  const char* err = nullptr;
+  st = fa::run_fwd(*p, false, reinterpret_cast<hipStream_t>(stream), &err, need > 0 ? workspace : nullptr);
+  if (st != FA_OK) return fail(st, err ? err : "launch failed");
+  return FA_OK;
+}
+
 fa_status fa_attention_varlen_fwd(const fa_fwd_params* p, void* stream) {
   g_last_error.clear();
   fa_status st = validate(p, /*varlen=*/true, /*fp8_ok=*/false, /*generic_ok=*/true);

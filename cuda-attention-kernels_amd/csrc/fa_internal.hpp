@@ -72,6 +72,7 @@ struct CombineArgs {
   int32_t hq, nq, n_split;
   int32_t group;       // q-heads per kv-head
   int32_t part_major;  // partial layout, as TileArgs::part_major
+  int64_t rows;  // prefill: B * Hq * Nq
 };
 
 // Number of rows (q-heads x queries) one split-K workgroup covers, and the
@@ -88,7 +89,15 @@ inline fa_status hip_status(hipError_t e, const char** err) {
 }
 
 // Launchers.  They assume fa_abi.cpp has validated `p`.
-fa_status run_fwd(const fa_fwd_params& p, bool varlen, hipStream_t stream, const char** err);
+fa_status run_fwd(const fa_fwd_params& p, bool varlen, hipStream_t stream, const char** err, void* workspace = nullptr);
+// Workspace run_fwd wants for a dense call (0: none; without one it runs unsplit).
+size_t fwd_workspace_bytes(const fa_fwd_params& p);
+// How run_fwd cuts a 16-bit call up: waves (of 32 queries) per workgroup, key splits per row block.
+struct FwdPlan {
+  int nw, n_split;
+};
+constexpr int kMaxFwdSplit = 32;
+FwdPlan plan_fwd(const fa_fwd_params& p, bool varlen, bool workspace);
 // fp32 at head dim 16 (fa_generic.hip); run_fwd forwards it here.
 fa_status run_fwd_generic(const fa_fwd_params& p, bool varlen, hipStream_t stream, const char** err);
 // fp32 at head dims 32 to 256 on the fp32 MFMA (fa_prefill_f32.hip); run_fwd forwards those here.

@@ -53,6 +53,8 @@ __device__ __forceinline__ void static_for(F&& f) {
   }
 }
 
+// a.n_split > 1 cuts a row block's key tiles over that many workgroups; each then writes an fp32
+// partial, and prefill_combine_kernel merges them (plan_fwd says when).
 template <int D, class E, int NW>
 __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2)))
 attn_fwd_kernel(const TileArgs a) {
@@ -107,7 +109,10 @@ attn_fwd_kernel(const TileArgs a) {
   }
   PrefillItem it;
   if (!prefill_item<D>(a, it)) return;  // grid padding (uniform over the workgroup)
-  const int b = it.b, hq = it.hq, kvh = it.kvh, rb = it.rb;
+  const int b = it.b, hq = it.hq, kvh = it.kvh;
+  // a.n_rowblk counts (row block, key split) pairs, the splits of a row block side by side
+  const int rb = a.n_split > 1 ? it.rb / a.n_split : it.rb;
+  const int sp = a.n_split > 1 ? it.rb - rb * a.n_split : 0;
 
   int seq_q = a.nq, seq_k = a.nk;
   int64_t qtok0 = 0, ktok0 = 0;
@@ -127,14 +132,24 @@ attn_fwd_kernel(const TileArgs a) {
 
   int khi = seq_k;
   if (a.causal) khi = min(khi, min(r0 + NW * 32, seq_q) - 1 + offset + 1);
-  const int n_tiles = khi > 0 ? (khi + BN - 1) / BN : 0;
-  // Tiles [0, n_fast) hold only keys that every query of the workgroup sees.
-  const int wg_mask_from = a.causal ? min(khi, r0 + offset + 1) : khi;
-  const int n_fast = wg_mask_from > 0 ? wg_mask_from / BN : 0;
+  int tile0 = 0;  // first tile of this workgroup's key range
+  if (a.n_split > 1) {
+    const int per = ((khi > 0 ? (khi + BN - 1) / BN : 0) + a.n_split - 1) / a.n_split;
+    tile0 = sp * per;
+    khi = min(khi, (tile0 + per) * BN);
+  }
 
   // ---- lane roles --------------------------------------------------------------------
   const int tid = (int)threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  // Tile t of this workgroup's key range starts at key0(t); local_tiles(n) of the call's first n
+  // tiles belong to it or to an earlier split.
+  auto key0 = [&](int t) __attribute__((always_inline)) { return (tile0 + t) * BN; };
+  auto local_tiles = [&](int n) __attribute__((always_inline)) { return max(n - tile0, 0); };
+  const int n_tiles = local_tiles(khi > 0 ? (khi + BN - 1) / BN : 0);
+  // Tiles [0, n_fast) hold only keys that every query of the workgroup sees.
+  const int wg_mask_from = a.causal ? min(khi, r0 + offset + 1) : khi;
+  const int n_fast = local_tiles(wg_mask_from > 0 ? wg_mask_from / BN : 0);
   const int g = lane >> 5, j = lane & 31;
   const int wr0 = r0 + wave * 32;
   const int qi = wr0 + j;
@@ -147,7 +162,7 @@ attn_fwd_kernel(const TileArgs a) {
   // before the workgroup's last row, and its later tiles hold only -inf scores (P = 0), so the
   // wave skips their compute and only issues its share of the DMA (with 8 waves up to 3 tiles).
   const int wave_khi = a.causal ? min(khi, min(wr0 + 32, seq_q) - 1 + offset + 1) : khi;
-  const int wave_tiles = wave_khi > 0 ? (wave_khi + BN - 1) / BN : 0;
+  const int wave_tiles = local_tiles(wave_khi > 0 ? (wave_khi + BN - 1) / BN : 0);
   const int qlim = qi + offset;  // last key this lane's row may see (causal)
 
   const uint8_t* kbase = (const uint8_t*)a.k + ((int64_t)b * a.skb + (int64_t)kvh * a.skh + ktok0 * a.skn) * 2;
@@ -212,9 +227,9 @@ attn_fwd_kernel(const TileArgs a) {
 
   // ---- prologue, first half: K_0, V_0, K_1 and then Q go out before the rest of the set-up
   if (n_tiles > 0) {
-    load_k(0, k_buf0);
-    load_v(0, v_buf0);
-    if (n_tiles > 1) load_k(BN, k_buf1);
+    load_k(key0(0), k_buf0);
+    load_v(key0(0), v_buf0);
+    if (n_tiles > 1) load_k(key0(1), k_buf1);
   }
   __builtin_amdgcn_sched_barrier(0);
   load_q();
@@ -413,7 +428,7 @@ attn_fwd_kernel(const TileArgs a) {
     l_run += rs;
     float mt = max_xor32(mx * c);
     if (t + 1 >= n_fast) {
-      const int n1 = (t + 1) * BN;
+      const int n1 = key0(t + 1);
       if (t + 1 < n_tiles) {
         if (n1 + BN > mask_from) {
           // an empty volatile asm cannot be speculated: without it the compiler
@@ -443,7 +458,7 @@ attn_fwd_kernel(const TileArgs a) {
     for (int kb = 0; kb < KB; ++kb) s_a[kb] = f32x16{};
 #pragma unroll
     for (int s = 0; s < KS; ++s) qk(k_buf0, s_a, s);
-    if (BN > mask_from) mask(s_a, 0);
+    if (key0(0) + BN > mask_from) mask(s_a, key0(0));
     update_max(tile_max(s_a));
     __syncthreads();  // every wave has read K_0: its buffer takes K_2
   }
@@ -459,9 +474,9 @@ attn_fwd_kernel(const TileArgs a) {
     auto& nxt = ST == 0 ? s_b : s_a;
     // K_{t+2} and V_{t+1} (zero-length descriptors past the last tile)
     if (NW == 4 || t < wave_tiles) {
-      body(k_next, v_this, cur, nxt, t, k_rsrc((t + 2) * BN), k_this, v_rsrc((t + 1) * BN), v_next);
+      body(k_next, v_this, cur, nxt, t, k_rsrc(key0(t + 2)), k_this, v_rsrc(key0(t + 1)), v_next);
     } else {
-      const __amdgpu_buffer_rsrc_t rk = k_rsrc((t + 2) * BN), rv = v_rsrc((t + 1) * BN);
+      const __amdgpu_buffer_rsrc_t rk = k_rsrc(key0(t + 2)), rv = v_rsrc(key0(t + 1));
 #pragma unroll
       for (int i = 0; i < QPW; ++i) dma_k(rk, k_this, i);
 #pragma unroll
@@ -476,18 +491,61 @@ attn_fwd_kernel(const TileArgs a) {
   }
 
   // ---- epilogue ------------------------------------------------------------------------
+  // Every wave has passed the last tile's barrier and its DMA has landed, so the K/V buffers are
+  // free for staging the output.
   if (!wave_active) return;
   // each lane summed its 16 of the row's keys per tile (or holds the full sum, MFMA_ROWSUM)
   const float l_tot = MFMA_ROWSUM ? l_acc[0] : sum_xor32(l_run);
+  if (a.n_split > 1) {
+    // fp32 partial of key split sp: O normalised by its own row sum (zeros for a row without keys
+    // here) and (m, l), [S][B, Hq, Nq][D]
+    const int64_t rows = (int64_t)a.kv_groups * a.group * seq_q;
+    const int64_t row0 = sp * rows + ((int64_t)b * a.hq + hq) * seq_q + wr0;
+    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    if (row_ok && g == 0) st8(a.ml + (row0 + j) * 2, __builtin_bit_cast(u32x2, f32x2{m_run, l_tot}));
+    if constexpr (NW * 32 * D * 4 <= 4 * TILE * 2) {
+      // through LDS, as the output below: whole rows per store instruction
+      constexpr int NCH = D / 4, REG = 32 * D * 4 / 2, PER_BUF = TILE / REG;
+      const int bi = wave / PER_BUF;
+      float* stage = (float*)((bi == 0 ? k_buf0 : bi == 1 ? k_buf1 : bi == 2 ? v_buf0 : v_buf1) + (wave % PER_BUF) * REG);
+#pragma unroll
+      for (int d = 0; d < DB; ++d) {
+#pragma unroll
+        for (int rq = 0; rq < 4; ++rq) {
+          if (d * 32 + 8 * rq >= D) continue;
+          const int c = 8 * d + 2 * rq + g;
+          *(f32x4*)(stage + j * D + ((c ^ (j & (NCH - 1))) * 4)) = f32x4{oacc[d][4 * rq] * inv, oacc[d][4 * rq + 1] * inv,
+                                                                         oacc[d][4 * rq + 2] * inv, oacc[d][4 * rq + 3] * inv};
+        }
+      }
+      constexpr int RPI = 64 / NCH;  // rows per 64-lane read
+      const int cc = lane % NCH;
+#pragma unroll
+      for (int i = 0; i < 32 / RPI; ++i) {
+        const int r = i * RPI + lane / NCH;
+        const u32x4 v = ld16(stage + r * D + ((cc ^ (r & (NCH - 1))) * 4));
+        if (wr0 + r < seq_q) st16((float*)a.o + (row0 + r) * D + cc * 4, v);
+      }
+    } else if (row_ok) {
+      float* op = (float*)a.o + (row0 + j) * D;
+#pragma unroll
+      for (int d = 0; d < DB; ++d) {
+#pragma unroll
+        for (int rq = 0; rq < 4; ++rq)
+          st16(op + d * 32 + 8 * rq + 4 * g, __builtin_bit_cast(u32x4, f32x4{oacc[d][4 * rq] * inv, oacc[d][4 * rq + 1] * inv,
+                                                                          oacc[d][4 * rq + 2] * inv, oacc[d][4 * rq + 3] * inv}));
+      }
+    }
+    return;
+  }
   // Rows that saw no key have l == 0 and emit zeros (triton_fwd.py:163-165).
   const float l_safe = (l_tot == 0.f) ? 1.f : l_tot;
   const float inv = 1.f / l_safe;
   // O is staged through LDS, row-major with 16-byte chunks XOR-swizzled by row, and written
   // back in whole rows: a lane of the O^T fragment holds 4 values of each of 16 chunks of one
   // row, so storing from the fragment sends each instruction to 32 rows (32 partial cache
-  // lines); from LDS, 16 consecutive lanes write one row's 256 bytes (D=128).  Every wave has
-  // passed the last tile's barrier and its DMA has landed, so the K/V buffers are free; each
-  // wave takes its own 32*D-element region of them.
+  // lines); from LDS, 16 consecutive lanes write one row's 256 bytes (D=128).  Each wave takes its
+  // own 32*D-element region of the K/V buffers.
   {
     constexpr int NCH = D / 8;                       // 16-byte chunks per row
     constexpr int SWZ = NCH < 16 ? NCH - 1 : 15;     // chunk swizzle by row
@@ -531,13 +589,159 @@ attn_fwd_kernel(const TileArgs a) {
   }
 }
 
+// Log-sum-exp merge of the key splits' partials: O = sum_s w_s O_s / sum_s w_s, w_s = 2^(m_s - m) l_s
+// (0 when no split saw a key).  A workgroup merges RPT rows of one (batch, q-head) per D/4 threads,
+// each thread 4 values of a row, so that consecutive lanes read consecutive 16-byte pieces; the
+// loads of CH splits are in flight together.
+constexpr int kCombineRows = 2;  // rows per thread
+
+template <int D, class E>
+__global__ void __launch_bounds__(256) prefill_combine_kernel(const CombineArgs c) {
+  constexpr int TPR = D / 4, RPT = kCombineRows, CH = 4;
+  constexpr float NEG_INF = -__builtin_inff();
+  const uint32_t rpw = (256 / TPR) * RPT, chunks = ((uint32_t)c.nq + rpw - 1) / rpw;
+  const uint32_t bh = blockIdx.x / chunks, chunk = blockIdx.x - bh * chunks;  // b * hq + head
+  const uint32_t b = bh / (uint32_t)c.hq, hq = bh - b * (uint32_t)c.hq;
+  const int dq = (int)threadIdx.x % TPR, r0 = (int)(chunk * rpw) + (int)threadIdx.x / TPR;
+  const int64_t rows = c.rows;
+  float m[RPT], l[RPT];
+  f32x4 acc[RPT];
+#pragma unroll
+  for (int i = 0; i < RPT; ++i) {
+    m[i] = NEG_INF;
+    l[i] = 0.f;
+    acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  for (int s0 = 0; s0 < c.n_split; s0 += CH) {
+    f32x2 st[CH][RPT];
+    f32x4 pv[CH][RPT];
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+#pragma unroll
+      for (int i = 0; i < RPT; ++i) {
+        const int qi = r0 + i * (256 / TPR);
+        st[u][i] = f32x2{NEG_INF, 0.f};
+        pv[u][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (s0 + u < c.n_split && qi < c.nq) {
+          const int64_t r = (s0 + u) * rows + (int64_t)bh * c.nq + qi;
+          st[u][i] = __builtin_bit_cast(f32x2, ld8(c.ml + 2 * r));
+          pv[u][i] = __builtin_bit_cast(f32x4, ld16(c.opart + r * D + 4 * dq));
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) {
+      float mn = m[i];
+#pragma unroll
+      for (int u = 0; u < CH; ++u) mn = fmaxf(mn, st[u][i][0]);
+      const float m_ref = (mn == NEG_INF) ? 0.f : mn;
+      const float alpha = fast_exp2(m[i] - m_ref);  // 0 while m = -inf
+      l[i] *= alpha;
+      acc[i] *= alpha;
+#pragma unroll
+      for (int u = 0; u < CH; ++u) {
+        const float w = fast_exp2(st[u][i][0] - m_ref) * st[u][i][1];
+        l[i] += w;
+        acc[i] += w * pv[u][i];
+      }
+      m[i] = mn;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < RPT; ++i) {
+    const int qi = r0 + i * (256 / TPR);
+    if (qi >= c.nq) continue;
+    const float l_safe = (l[i] == 0.f) ? 1.f : l[i];
+    const float inv = 1.f / l_safe;
+    if (c.lse != nullptr && dq == 0) c.lse[b * c.slb + (int64_t)hq * c.slh + qi] = (m[i] + __log2f(l_safe)) * kLn2;
+    uint16_t* o = (uint16_t*)c.o + b * c.sob + (int64_t)hq * c.soh + (int64_t)qi * c.son + 4 * dq;
+    st8(o, u32x2{pack2<E>(acc[i][0] * inv, acc[i][1] * inv), pack2<E>(acc[i][2] * inv, acc[i][3] * inv)});
+  }
+}
+
+template <int D, class E>
+static hipError_t launch_prefill_combine(const CombineArgs& c, int64_t heads, hipStream_t stream) {
+  constexpr int RPW = 1024 / D * kCombineRows;
+  hipLaunchKernelGGL((prefill_combine_kernel<D, E>), dim3((unsigned)(heads * ((c.nq + RPW - 1) / RPW))), dim3(256), 0,
+                     stream, c);
+  return hipGetLastError();
+}
+
 template <int D, class E, int NW>
 static hipError_t launch_fwd(const TileArgs& a, hipStream_t stream) {
   hipLaunchKernelGGL((attn_fwd_kernel<D, E, NW>), dim3((unsigned)a.total), dim3(NW * 64), 0, stream, a);
   return hipGetLastError();
 }
 
-fa_status run_fwd(const fa_fwd_params& p, bool varlen, hipStream_t stream, const char** err) {
+template <int D, class E>
+static hipError_t launch_fwd_plan(const TileArgs& a, const FwdPlan& plan, hipStream_t stream) {
+  if constexpr (D == 128) {
+    if (plan.nw == 8) return launch_fwd<D, E, 8>(a, stream);
+  }
+  return launch_fwd<D, E, 4>(a, stream);
+}
+
+FwdPlan plan_fwd(const fa_fwd_params& p, bool varlen, bool workspace) {
+  constexpr int kCus = 256;  // compute units of an MI355X
+  const int d = p.head_dim;
+  const int nq = varlen ? p.max_seqlen_q : p.seqlen_q, nk = varlen ? p.max_seqlen_k : p.seqlen_k;
+  // Dense D=128 with at least 4096 queries (2048 without the causal mask) runs 8 waves (256
+  // queries) per workgroup: each K/V tile feeds twice the rows, halving the DMA per MFMA
+  // (measured over 4 waves, Hq=32 Hkv=8: +1% causal at N=4096, +2% at 8192 and 16384, +1.7%
+  // non-causal at 2048).  Shorter sequences keep 4 (more, shorter workgroups whose start
+  // overlaps the other workgroup on the CU: 8 waves lose 5% causal at N=1024, 2.5% at 2048,
+  // 0.7% non-causal at 1024).  D=64 keeps 4 (-3% with 8) and D=256 runs one wave per SIMD.
+  // Varlen applies the same rule to its longest sequence (max_seqlen_q): a causal batch of 16
+  // sequences of 0-4073 tokens keeps 4 waves, and 8 from 2048 measured 2-5% slower on it (its
+  // short sequences leave more of a 256-query block empty).  A wave computes the same tiles
+  // in the same order with 4 or 8 waves per workgroup, so the result does not depend on the
+  // choice.
+  FwdPlan plan{};
+  plan.nw = (d == 128 && nq >= (p.causal ? 4096 : 2048)) ? 8 : 4;
+  plan.n_split = 1;
+
+  // Key splits: a call whose row blocks leave compute units idle (few queries against many keys)
+  // cuts each block's keys over several workgroups.  The estimate below, in microseconds, charges
+  // a CU 1.0 per 128-query tile it runs with two waves per SIMD, 1.15 with one, 0.8 at D=256 (whose
+  // workgroups run one per CU); the partials 0.4 per MB (written and read back) and the second
+  // launch 10 (4 on the GPU, the rest on the host).  512 queries against 16384 keys (Hq=32 Hkv=8
+  // D=128 causal, 128 row blocks): 223 us unsplit, 132 with 4 splits of 256-query blocks (8
+  // splits: 143 with 128-query blocks); 64 queries against 33000: 441 -> 68; 1000 queries against
+  // 3000 (256 row blocks) stay unsplit at 52 (2 splits: 58).
+  const int64_t heads = (int64_t)p.batch * p.heads_q;
+  const int bn = d <= 64 ? 128 : (d == 256 ? 32 : 64);
+  if (varlen || !workspace || nk <= 0 || heads * ((nq + 127) / 128) > kCus) return plan;
+  const double tiles = (nk + bn - 1) / bn;  // of the last (heaviest) row block
+  // mean over the row blocks: a causal first block sees nk - nq + 128 keys
+  const double mean = p.causal ? 0.5 * (tiles + std::max(1.0, (double)(nk - nq + 128) / bn)) : tiles;
+  auto cost = [&](int nw, int s) {
+    const int64_t wgs = heads * ((nq + nw * 32 - 1) / (nw * 32)) * s;
+    const double per_cu = (double)((wgs + kCus - 1) / kCus);
+    const double tile = d == 256 ? 0.8 : nw == 8 ? 2.0 : per_cu > 1 ? 1.0 : 1.15;
+    const double partials = s > 1 ? 10.0 + 0.4e-6 * (double)(heads * nq) * s * d * 4 : 0.0;
+    return tile * std::max(tiles, per_cu * mean) / s + partials;
+  };
+  double best = 0.95 * cost(4, 1);
+  for (int nw = 4; nw <= (d == 128 && nq > 128 ? 8 : 4); nw += 4) {
+    for (int s = 2; s <= kMaxFwdSplit && s * 4 <= tiles; s *= 2) {
+      if (cost(nw, s) < best) {
+        best = cost(nw, s);
+        plan.nw = nw;
+        plan.n_split = s;
+      }
+    }
+  }
+  return plan;
+}
+
+size_t fwd_workspace_bytes(const fa_fwd_params& p) {
+  if (p.dtype != FA_DTYPE_BF16 && p.dtype != FA_DTYPE_F16) return 0;
+  const FwdPlan plan = plan_fwd(p, false, true);
+  if (plan.n_split <= 1) return 0;
+  return (size_t)p.batch * p.heads_q * p.seqlen_q * plan.n_split * ((size_t)p.head_dim + 2) * sizeof(float);
+}
+
+fa_status run_fwd(const fa_fwd_params& p, bool varlen, hipStream_t stream, const char** err, void* workspace) {
   const bool mfma = (p.dtype == FA_DTYPE_BF16 || p.dtype == FA_DTYPE_F16) &&
                     (p.head_dim == 16 || p.head_dim == 32 || p.head_dim == 64 || p.head_dim == 128 ||
                      p.head_dim == 256);
@@ -563,19 +767,13 @@ fa_status run_fwd(const fa_fwd_params& p, bool varlen, hipStream_t stream, const
     a.sqb = a.skb = a.svb = a.sob = a.slb = 0;  // rows are addressed by packed token index
   }
   if (a.nq <= 0 || p.batch <= 0) return FA_OK;
-  // Dense D=128 with at least 4096 queries (2048 without the causal mask) runs 8 waves (256
-  // queries) per workgroup: each K/V tile feeds twice the rows, halving the DMA per MFMA
-  // (measured over 4 waves, Hq=32 Hkv=8: +1% causal at N=4096, +2% at 8192 and 16384, +1.7%
-  // non-causal at 2048).  Shorter sequences keep 4 (more, shorter workgroups whose start
-  // overlaps the other workgroup on the CU: 8 waves lose 5% causal at N=1024, 2.5% at 2048,
-  // 0.7% non-causal at 1024).  D=64 keeps 4 (-3% with 8) and D=256 runs one wave per SIMD.
-  // Varlen applies the same rule to its longest sequence (max_seqlen_q): a causal batch of 16
-  // sequences of 0-4073 tokens keeps 4 waves, and 8 from 2048 measured 2-5% slower on it (its
-  // short sequences leave more of a 256-query block empty).  A wave computes the same tiles
-  // in the same order with 4 or 8 waves per workgroup, so the result does not depend on the
-  // choice.
-  const int nw = (p.head_dim == 128 && a.nq >= (p.causal ? 4096 : 2048)) ? 8 : 4;
-  a.n_rowblk = (a.nq + nw * 32 - 1) / (nw * 32);
+  const FwdPlan plan = plan_fwd(p, varlen, workspace != nullptr);
+  const int64_t rows = (int64_t)p.batch * p.heads_q * a.nq;
+  if (plan.n_split > 1) {
+    a.o = workspace;
+    a.ml = (float*)workspace + rows * plan.n_split * p.head_dim;
+  }
+  a.n_rowblk = (a.nq + plan.nw * 32 - 1) / (plan.nw * 32) * plan.n_split;
   const int64_t kv_groups = (int64_t)p.batch * p.heads_kv;
   // varlen: the (sequence, kv-head) groups are padded to a multiple of the 8 XCDs
   const int64_t groups = varlen ? (kv_groups + 7) / 8 * 8 : kv_groups;
@@ -589,24 +787,41 @@ fa_status run_fwd(const fa_fwd_params& p, bool varlen, hipStream_t stream, const
   // a unit never holds more than the (batch, q-head) pairs there are, which keeps u_items <= total
   a.u_heads = (int32_t)std::min<int64_t>(prefill_unit_heads(a.nk, p.head_dim, a.group), kv_groups * a.group);
   a.u_items = a.u_heads * a.n_rowblk;
-  a.n_split = 1;
-  a.split_len = 0;
+  a.n_split = plan.n_split;
   hipError_t e = hipErrorInvalidValue;
   const bool bf = p.dtype == FA_DTYPE_BF16;
-  if (p.head_dim == 128) {
-    if (nw == 8) {
-      e = bf ? launch_fwd<128, BF16, 8>(a, stream) : launch_fwd<128, F16, 8>(a, stream);
-    } else {
-      e = bf ? launch_fwd<128, BF16, 4>(a, stream) : launch_fwd<128, F16, 4>(a, stream);
-    }
-  } else if (p.head_dim == 64) {
-    e = bf ? launch_fwd<64, BF16, 4>(a, stream) : launch_fwd<64, F16, 4>(a, stream);
-  } else if (p.head_dim == 32) {
-    e = bf ? launch_fwd<32, BF16, 4>(a, stream) : launch_fwd<32, F16, 4>(a, stream);
-  } else if (p.head_dim == 16) {
-    e = bf ? launch_fwd<16, BF16, 4>(a, stream) : launch_fwd<16, F16, 4>(a, stream);
-  } else if (p.head_dim == 256) {
-    e = bf ? launch_fwd<256, BF16, 4>(a, stream) : launch_fwd<256, F16, 4>(a, stream);
+  switch (p.head_dim) {
+    case 128: e = bf ? launch_fwd_plan<128, BF16>(a, plan, stream) : launch_fwd_plan<128, F16>(a, plan, stream); break;
+    case 64: e = bf ? launch_fwd_plan<64, BF16>(a, plan, stream) : launch_fwd_plan<64, F16>(a, plan, stream); break;
+    case 32: e = bf ? launch_fwd_plan<32, BF16>(a, plan, stream) : launch_fwd_plan<32, F16>(a, plan, stream); break;
+    case 16: e = bf ? launch_fwd_plan<16, BF16>(a, plan, stream) : launch_fwd_plan<16, F16>(a, plan, stream); break;
+    case 256: e = bf ? launch_fwd_plan<256, BF16>(a, plan, stream) : launch_fwd_plan<256, F16>(a, plan, stream); break;
+    default: break;
+  }
+  if (e != hipSuccess || plan.n_split == 1) return hip_status(e, err);
+
+  const int64_t heads = (int64_t)p.batch * p.heads_q;
+  CombineArgs c{};
+  c.rows = rows;
+  c.opart = (const float*)a.o;
+  c.ml = a.ml;
+  c.o = p.o;
+  c.sob = p.o_stride_b;
+  c.soh = p.o_stride_h;
+  c.son = p.o_stride_n;
+  c.hq = p.heads_q;
+  c.nq = p.seqlen_q;
+  c.n_split = plan.n_split;
+  c.lse = p.lse;
+  c.slb = p.lse_stride_b;
+  c.slh = p.lse_stride_h;
+  switch (p.head_dim) {
+    case 128: e = bf ? launch_prefill_combine<128, BF16>(c, heads, stream) : launch_prefill_combine<128, F16>(c, heads, stream); break;
+    case 64: e = bf ? launch_prefill_combine<64, BF16>(c, heads, stream) : launch_prefill_combine<64, F16>(c, heads, stream); break;
+    case 32: e = bf ? launch_prefill_combine<32, BF16>(c, heads, stream) : launch_prefill_combine<32, F16>(c, heads, stream); break;
+    case 16: e = bf ? launch_prefill_combine<16, BF16>(c, heads, stream) : launch_prefill_combine<16, F16>(c, heads, stream); break;
+    case 256: e = bf ? launch_prefill_combine<256, BF16>(c, heads, stream) : launch_prefill_combine<256, F16>(c, heads, stream); break;
+    default: break;
   }
   return hip_status(e, err);
 }

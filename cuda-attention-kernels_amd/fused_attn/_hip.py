@@ -135,6 +135,10 @@ def _bind(lib: ctypes.CDLL) -> None:
     P = ctypes.POINTER(FwdParams)
     lib.fa_attention_fwd.argtypes = [P, ctypes.c_void_p]
     lib.fa_attention_fwd.restype = ctypes.c_int
+    lib.fa_attention_fwd_workspace_bytes.argtypes = [P]
+    lib.fa_attention_fwd_workspace_bytes.restype = ctypes.c_size_t
+    lib.fa_attention_fwd_ws.argtypes = [P, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+    lib.fa_attention_fwd_ws.restype = ctypes.c_int
     lib.fa_attention_varlen_fwd.argtypes = [P, ctypes.c_void_p]
     lib.fa_attention_varlen_fwd.restype = ctypes.c_int
     lib.fa_splitk_workspace_bytes.argtypes = [ctypes.c_int32] * 5
@@ -433,8 +437,10 @@ def fwd(q, k, v, causal: bool = False, scale: Optional[float] = None, return_lse
     o = _new_output(q) if out is None else out
     lse = torch.empty(q.shape[:3], dtype=torch.float32, device=q.device) if return_lse else None
     p = make_params(q, k, v, o, causal, scale, lse=lse)
+    need = lib.fa_attention_fwd_workspace_bytes(p)
+    ws = torch.empty(need // 4, dtype=torch.float32, device=q.device) if need else None
     with _on_device(q.device):
-        _check(lib.fa_attention_fwd(ctypes.byref(p), ctypes.c_void_p(_stream(q))), "attention_fwd")
+        _check(lib.fa_attention_fwd_ws(p, ws.data_ptr() if need else None, need, _stream(q)), "attention_fwd")
     return (o, lse) if return_lse else o
 
 

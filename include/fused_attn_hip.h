@@ -100,6 +100,15 @@ typedef struct fa_fwd_params {
    on the generic fp32-math kernel at D = 16.  D in {16, 32, 64, 128, 256}. */
 fa_status fa_attention_fwd(const fa_fwd_params* p, void* stream);
 
+/* Bytes of workspace fa_attention_fwd_ws wants for these parameters: 0 for a grid that fills the GPU
+   by itself, else room for the fp32 partials of the key splits it is cut into (o, (max, sum)). */
+size_t fa_attention_fwd_workspace_bytes(const fa_fwd_params* p);
+
+/* fa_attention_fwd with a caller workspace of at least fa_attention_fwd_workspace_bytes (16-byte
+   aligned; may be NULL when that is 0).  Few queries against many keys leave most compute units
+   idle; the key range is then cut over workgroups and a second kernel merges the partials. */
+fa_status fa_attention_fwd_ws(const fa_fwd_params* p, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Packed variable-length forward.  Replaces attention_varlen_triton
    (fused_attn/triton_fwd.py:268-309).  Needs cu_seqlens_q/k and max_seqlen_q; optional LSE. */
 fa_status fa_attention_varlen_fwd(const fa_fwd_params* p, void* stream);
