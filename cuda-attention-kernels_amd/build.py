@@ -36,6 +36,13 @@ COMMON = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 
+# MFMA accumulators in VGPRs for the sources whose D=256 kernels need more than 256 registers: by itself the
+# compiler keeps those accumulators in AGPRs and copies them to VGPRs and back around the softmax rescale
+# (D=256, B=16 Hq=64 Hkv=8: FP8 decode over 16384 keys 271 -> 234 us; fp32 prefill, 2 x 4 heads, 2048 x 2048:
+# 630 -> 601).  The 16-bit prefill keeps the default: it measured 5-7% slower at D=256 with it.
+VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
+EXTRA = {"fa_splitk.hip": VGPR_FORM, "fa_prefill_f32.hip": VGPR_FORM}
+
 
 def _run(cmd: list[str]) -> None:
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -55,7 +62,7 @@ def build(verbose: bool = False) -> str:
         objs = []
         for src in sources:
             obj = os.path.join(BUILD_DIR, os.path.splitext(src)[0] + ".o")
-            cmds.append([HIPCC, *COMMON, "-x", "hip", "-c", os.path.join(CSRC, src), "-o", obj])
+            cmds.append([HIPCC, *COMMON, *EXTRA.get(src, []), "-x", "hip", "-c", os.path.join(CSRC, src), "-o", obj])
             objs.append(obj)
         return objs
 
