@@ -51,6 +51,7 @@ struct TileArgs {
   // (partition-major: the rows one workgroup writes for one partition are one block)
   int32_t part_major;
   int32_t o16;  // prefill: O base and strides allow 16-byte stores
+  int32_t batch, n_items;  // paged split-K: sequences, and batch * hkv * n_chunk
   int32_t u_heads, u_items;  // dense prefill schedule: q-heads per scheduling unit, and times n_rowblk
 };
 
@@ -73,6 +74,8 @@ struct CombineArgs {
   int32_t group;       // q-heads per kv-head
   int32_t part_major;  // partial layout, as TileArgs::part_major
   int64_t rows;  // prefill: B * Hq * Nq
+  const int32_t* seqlens_k;  // paged: the sequences' lengths (clamped to [0, nk])
+  int32_t nk, split_len;
 };
 
 // Number of rows (q-heads x queries) one split-K workgroup covers, and the
