@@ -51,6 +51,8 @@ struct TileArgs {
   // (partition-major: the rows one workgroup writes for one partition are one block)
   int32_t part_major;
   int32_t o16;  // prefill: O base and strides allow 16-byte stores
+  // dense prefill: pair heavy and light workgroups on a CU; deal the workgroups to the XCDs
+  int32_t fold, deal;
   int32_t batch, n_items;  // paged split-K: sequences, and batch * hkv * n_chunk
   int32_t u_heads, u_items;  // dense prefill schedule: q-heads per scheduling unit, and times n_rowblk
 };
