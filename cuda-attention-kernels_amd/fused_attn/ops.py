@@ -10,7 +10,7 @@ ops.py:34-73, collapse into these two):
 
 * GPU tensors go to the HIP backend (``_hip``): MFMA FA2 prefill, or split-K
   flash-decoding for decode-shaped calls (at most 16 queries against at least
-  2048 keys, ops.py:36-37,63-66).  If the HIP library cannot run on the device
+  2048 keys, ops.py:36-37,63-66; grouped heads with few rows from 512 or 192).  If the HIP library cannot run on the device
   the call raises; it never falls back silently.
 * CPU tensors, or ``FUSED_ATTN_BACKEND=reference``, use the unfused PyTorch
   path in ``reference.py``.
@@ -74,6 +74,29 @@ SPLITK_DTYPES = (torch.float16, torch.bfloat16)  # the split-K kernel: 16-bit Q 
 SPLITK_HEAD_DIMS = (64, 128, 256)
 
 
+def _is_short_decode(q: torch.Tensor, k: torch.Tensor) -> bool:
+    """Decode steps against contexts below SPLITK_MIN_K that split-K still serves faster.
+
+    The prefill kernel gives every q-head a 128-row block and reads the K/V of a GQA group once per q-head;
+    split-K takes the up to 32 (q-head, query) rows of a kv-head as one wave's rows and reads it once, but needs
+    a second launch.  GPU time, us, prefill kernel and split-K, D=128 bf16 Hq=32 Hkv=8, one query: 16 sequences
+    of 1000 keys 33.0 and 18.3, 40 of 256 keys 27.4 and 15.9, one of 700 keys 15.4 and 11.3; but one of 400 keys
+    at D=64 10.2 and 10.8, and 10 of 700 keys with 16 queries (64 rows) 23.7 and 31.2.  Without grouped heads
+    nothing is read twice: only a few heads, which leave the GPU idle, gain (32 heads, 700 keys 15.3 and 11.3).
+    At D=256 a small call stays with the prefill kernel (32 heads, 1200 keys 14.4 and 17.2)."""
+    if q.dim() != 4 or k.dim() != 4 or k.shape[1] == 0 or q.shape[1] % k.shape[1] != 0:
+        return False
+    b, hq, nq, d = q.shape
+    nk, group, heads = k.shape[2], hq // k.shape[1], b * hq
+    if nq == 0 or group * nq > 32:
+        return False
+    if group == 1:
+        return nk >= 512 and heads <= 128 and nq <= 4 and d != 256
+    if heads > (256 if d == 256 else 512):
+        return nk >= 192
+    return nk >= 512 and (d != 256 or heads > 64)
+
+
 def _hip_kernel_for(q: torch.Tensor, k: torch.Tensor) -> str:
     """Which HIP kernel family serves this call: ``splitk`` or ``fwd``.
 
@@ -82,7 +105,7 @@ def _hip_kernel_for(q: torch.Tensor, k: torch.Tensor) -> str:
     """
     if q.dtype not in SPLITK_DTYPES or q.shape[-1] not in SPLITK_HEAD_DIMS:
         return "fwd"
-    if os.environ.get("FUSED_ATTN_BACKEND") == "splitk" or is_decode_shaped(q, k):
+    if os.environ.get("FUSED_ATTN_BACKEND") == "splitk" or is_decode_shaped(q, k) or _is_short_decode(q, k):
         return "splitk"
     return "fwd"
 
