@@ -6,7 +6,8 @@
 // (triton_fwd.py:169-172).  Both products run on v_mfma_f32_32x32x2_f32, so every product
 // and sum is an fp32 operation, and P stays fp32.
 //
-// A workgroup of 4 waves covers 128 queries of one q-head; wave w owns 32 of them.  K and V
+// A workgroup of 4 waves covers 128 queries of one q-head; wave w owns 32 of them (in small grids 32 queries,
+// the key tiles shared out among the waves: KS below).  K and V
 // stream through LDS in 32-key fp32 tiles, double-buffered and filled straight from memory.
 //
 // Operand layout per 32-key block and wave (lane l: j = l % 32, g = l / 32):
@@ -28,6 +29,8 @@
 //    4-byte reads, small beside the 64-cycle MFMAs they feed).
 #include <float.h>
 
+#include <algorithm>
+
 #include <type_traits>
 
 #include "fa_device.hpp"
@@ -41,13 +44,17 @@ __device__ __forceinline__ f32x16 mfma_f32(float a, float b, const f32x16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
-template <int D>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2)))
+// KS (D <= 128): a workgroup covers 32 queries and its waves share out the key tiles, wave w taking tiles w,
+// w + 4, ... through LDS of its own, without barriers; the four partial results are merged through LDS at
+// the end.  Four times the workgroups with a quarter of the serial chain each (run_fwd_f32 says when).
+template <int D, bool KS>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 || (KS && D >= 64) ? 1 : 2)))
 attn_fwd_f32_kernel(const TileArgs a) {
   constexpr int NW = 4;
   constexpr int BN = 32;                      // keys per tile: one 32-key MFMA block
   constexpr int TILE = BN * D;                // floats per K (or V) tile
-  constexpr int QPW = TILE * 4 / 1024 / NW;   // 1-KiB DMA blocks per wave per tile
+  constexpr int RPB = KS ? 32 : NW * 32;      // queries per workgroup
+  constexpr int QPW = TILE * 4 / 1024 / (KS ? 1 : NW);  // 1-KiB DMA blocks per wave per tile
   constexpr int DB = D / 32;                  // 32-row d blocks of O^T
   constexpr int HS = D / 2;                   // k = 2 steps of S^T
   static_assert(D == 32 || D == 64 || D == 128 || D == 256, "head dim");
@@ -55,16 +62,21 @@ attn_fwd_f32_kernel(const TileArgs a) {
   constexpr float NEG_INF = -__builtin_inff();
 
   // separate arrays so that the compiler can tell a DMA into one buffer from reads of another
-  __shared__ __align__(16) float k_buf0[TILE];
-  __shared__ __align__(16) float k_buf1[TILE];
-  __shared__ __align__(16) float v_buf0[TILE];
-  __shared__ __align__(16) float v_buf1[TILE];
+  // (KS: a buffer holds one tile per wave; at D=128 one stage of them fills 128 KiB)
+  static_assert(!KS || D <= 128, "a tile per wave must fit LDS");
+  constexpr bool TWO_STAGES = !KS || D <= 64;
+  constexpr int BUF = KS ? NW * TILE : TILE;
+  __shared__ __align__(16) float k_buf0[BUF];
+  __shared__ __align__(16) float k_buf1[TWO_STAGES ? BUF : 4];
+  __shared__ __align__(16) float v_buf0[BUF];
+  __shared__ __align__(16) float v_buf1[TWO_STAGES ? BUF : 4];
 
   // ---- work item: (batch or sequence, q-head, 128-query block), rank-major ---------------
   // All (batch, q-head) pairs at one rank run together (heaviest causal blocks first), the
-  // q-heads of one kv-head side by side; xcd_remap gives each XCD a contiguous range.
+  // q-heads of one kv-head side by side; xcd_remap gives each XCD a contiguous range.  Causal ranks
+  // are dealt to the XCDs instead: a contiguous range gave the first XCD all the heaviest.
   const int nbh = a.total / a.n_rowblk;
-  const int logical = xcd_remap((int)blockIdx.x, a.total);
+  const int logical = a.causal ? (int)blockIdx.x : xcd_remap((int)blockIdx.x, a.total);
   const int mrev = logical / nbh;
   const int item = logical % nbh;
   const int hq = item % a.hq;
@@ -82,18 +94,18 @@ attn_fwd_f32_kernel(const TileArgs a) {
     qtok0 = qs;
     ktok0 = ks;
   }
-  const int r0 = rb * NW * 32;
+  const int r0 = rb * RPB;
   if (r0 >= seq_q) return;  // uniform over the workgroup (zero-length sequences exit here)
   const int offset = seq_k - seq_q;  // bottom-right causal alignment (reference.py:24-33)
   int khi = seq_k;
-  if (a.causal) khi = min(khi, min(r0 + NW * 32, seq_q) + offset);
+  if (a.causal) khi = min(khi, min(r0 + RPB, seq_q) + offset);
   const int n_tiles = khi > 0 ? (khi + BN - 1) / BN : 0;
 
   // ---- lane roles --------------------------------------------------------------------
   const int tid = (int)threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int g = lane >> 5, j = lane & 31;
-  const int wr0 = r0 + wave * 32;
+  const int wr0 = KS ? r0 : r0 + wave * 32;
   const int qi = wr0 + j;
   const bool row_ok = qi < seq_q;
   const bool wave_active = wr0 < seq_q;
@@ -139,7 +151,7 @@ attn_fwd_f32_kernel(const TileArgs a) {
     const __amdgpu_buffer_rsrc_t rv = make_rsrc(vbase + (int64_t)n0 * vrow_bytes, limit(n0, vrow_bytes));
 #pragma unroll
     for (int i = 0; i < QPW; ++i) {
-      const int blk = wave * QPW + i;
+      const int blk = (KS ? 0 : wave * QPW) + i;  // within the tile (KS: the wave's own)
       const int byte = blk * 1024 + lane * 16;
       const int r = byte / (D * 4), p = (byte % (D * 4)) / 16;
       lds_dma16<false>(rk, (uint8_t*)kd + blk * 1024, r * (int)krow_bytes + ((p ^ swz(r)) * 16));
@@ -220,21 +232,99 @@ attn_fwd_f32_kernel(const TileArgs a) {
   };
 
   // ---- main loop, unrolled by 2 so that every buffer is named at compile time ------------
-  if (n_tiles > 0) load_tiles(0, k_buf0, v_buf0);
-  auto step = [&](auto stage_tag, int t) __attribute__((always_inline)) {
-    constexpr int ST = decltype(stage_tag)::value;
-    const float* kc = ST == 0 ? k_buf0 : k_buf1;  // holds tile t
-    const float* vc = ST == 0 ? v_buf0 : v_buf1;
-    float* kn = ST == 0 ? k_buf1 : k_buf0;  // held tile t-1 (every wave is done with it), takes t+1
-    float* vn = ST == 0 ? v_buf1 : v_buf0;
-    lds_dma_wait();
+  if constexpr (KS) {
+    const int own = wave * TILE;
+    if constexpr (TWO_STAGES) {
+      if (wave < n_tiles) load_tiles(wave * BN, k_buf0 + own, v_buf0 + own);
+      auto step = [&](auto stage_tag, int t) __attribute__((always_inline)) {
+        constexpr int ST = decltype(stage_tag)::value;
+        lds_dma_wait();
+        __asm__ volatile("" ::: "memory");
+        // (the stage of tile t - 4 was read before that tile's last MFMAs issued)
+        if (t + NW < n_tiles) load_tiles((t + NW) * BN, (ST == 0 ? k_buf1 : k_buf0) + own, (ST == 0 ? v_buf1 : v_buf0) + own);
+        tile((ST == 0 ? k_buf0 : k_buf1) + own, (ST == 0 ? v_buf0 : v_buf1) + own, t * BN);
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the stage has been read
+        __asm__ volatile("" ::: "memory");
+      };
+      for (int t = wave; t < n_tiles; t += 2 * NW) {
+        step(std::integral_constant<int, 0>{}, t);
+        if (t + NW < n_tiles) step(std::integral_constant<int, 1>{}, t + NW);
+      }
+    } else {
+      for (int t = wave; t < n_tiles; t += NW) {
+        load_tiles(t * BN, k_buf0 + own, v_buf0 + own);
+        lds_dma_wait();
+        __asm__ volatile("" ::: "memory");
+        tile(k_buf0 + own, v_buf0 + own, t * BN);
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the stage has been read
+        __asm__ volatile("" ::: "memory");
+      }
+    }
+  } else {
+    if (n_tiles > 0) load_tiles(0, k_buf0, v_buf0);
+    auto step = [&](auto stage_tag, int t) __attribute__((always_inline)) {
+      constexpr int ST = decltype(stage_tag)::value;
+      const float* kc = ST == 0 ? k_buf0 : k_buf1;  // holds tile t
+      const float* vc = ST == 0 ? v_buf0 : v_buf1;
+      float* kn = ST == 0 ? k_buf1 : k_buf0;  // held tile t-1 (every wave is done with it), takes t+1
+      float* vn = ST == 0 ? v_buf1 : v_buf0;
+      lds_dma_wait();
+      __syncthreads();
+      if (t + 1 < n_tiles) load_tiles((t + 1) * BN, kn, vn);
+      if (t * BN < wave_khi) tile(kc, vc, t * BN);
+    };
+    for (int t = 0; t < n_tiles; t += 2) {
+      step(std::integral_constant<int, 0>{}, t);
+      if (t + 1 < n_tiles) step(std::integral_constant<int, 1>{}, t + 1);
+    }
+  }
+
+  if constexpr (KS) {
+    // ---- merge: O = sum_w 2^(m_w - m) O_w / sum_w 2^(m_w - m) l_w over the waves ------------
+    // O_w goes to the wave's own K buffer as rows of D floats, 16-byte chunks XOR-swizzled by row: lane
+    // (j, g) holds columns DB*(8q + 4g) .. + 4*DB - 1 of row j in registers 4q..4q+3 of its DB blocks.
+    constexpr int NCH = D / 4;
+    __shared__ f32x2 ml[NW][32];
+    const float l_w = sum_xor32(l_run);
+    float* part = k_buf0 + wave * TILE;
+#pragma unroll
+    for (int q4 = 0; q4 < 4; ++q4) {
+#pragma unroll
+      for (int cc = 0; cc < DB; ++cc) {
+        f32x4 w;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = oacc[(4 * cc + e) % DB][4 * q4 + (4 * cc + e) / DB];
+        *(f32x4*)(part + j * D + (((DB * (2 * q4 + g) + cc) ^ (j & (NCH - 1))) * 4)) = w;
+      }
+    }
+    if (g == 0) ml[wave][j] = f32x2{m_run, l_w};
     __syncthreads();
-    if (t + 1 < n_tiles) load_tiles((t + 1) * BN, kn, vn);
-    if (t * BN < wave_khi) tile(kc, vc, t * BN);
-  };
-  for (int t = 0; t < n_tiles; t += 2) {
-    step(std::integral_constant<int, 0>{}, t);
-    if (t + 1 < n_tiles) step(std::integral_constant<int, 1>{}, t + 1);
+#pragma unroll
+    for (int i = 0; i < 32 * NCH / 256; ++i) {
+      const int idx = tid + 256 * i, row = idx / NCH, ch = idx % NCH;
+      f32x2 st[NW];
+#pragma unroll
+      for (int w = 0; w < NW; ++w) st[w] = ml[w][row];
+      const float m = vmax(vmax(st[0][0], st[1][0]), vmax(st[2][0], st[3][0]));
+      const float m_ref = (m == NEG_INF) ? 0.f : m;
+      float l = 0.f;
+      f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const float f = fast_exp2(st[w][0] - m_ref);  // 0 for a wave that saw no key of this row
+        l += f * st[w][1];
+        o += f * *(const f32x4*)(k_buf0 + w * TILE + row * D + ((ch ^ (row & (NCH - 1))) * 4));
+      }
+      if (r0 + row >= seq_q) continue;
+      const float l_safe = (l == 0.f) ? 1.f : l;
+      const float inv = 1.f / l_safe;
+      float* op = (float*)a.o + (int64_t)b * a.sob + (int64_t)hq * a.soh + (qtok0 + r0 + row) * a.son + 4 * ch;
+      st8(op, __builtin_bit_cast(u32x2, f32x2{o[0] * inv, o[1] * inv}));
+      st8(op + 2, __builtin_bit_cast(u32x2, f32x2{o[2] * inv, o[3] * inv}));
+      if (a.lse != nullptr && ch == 0)
+        a.lse[(int64_t)b * a.slb + (int64_t)hq * a.slh + (qtok0 + r0 + row)] = (m + __log2f(l_safe)) * kLn2;
+    }
+    return;
   }
 
   // ---- epilogue ------------------------------------------------------------------------
@@ -264,12 +354,37 @@ attn_fwd_f32_kernel(const TileArgs a) {
 }
 
 template <int D>
-hipError_t launch_f32(const TileArgs& a, hipStream_t stream) {
-  hipLaunchKernelGGL((attn_fwd_f32_kernel<D>), dim3((unsigned)a.total), dim3(256), 0, stream, a);
+hipError_t launch_f32(const TileArgs& a, bool key_split, hipStream_t stream) {
+  if constexpr (D <= 128) {
+    if (key_split) {
+      hipLaunchKernelGGL((attn_fwd_f32_kernel<D, true>), dim3((unsigned)a.total), dim3(256), 0, stream, a);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((attn_fwd_f32_kernel<D, false>), dim3((unsigned)a.total), dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 
 }  // namespace
+
+// Whether a workgroup per 32 queries with the keys shared out among its waves (KS) beats one per 128 queries.
+// Both in units of one 32-key tile of a 4-wave workgroup, per compute unit: the plain kernel takes its
+// heaviest row block or the mean load of the 256 CUs, whichever is longer; KS takes a quarter of the tiles, 10%
+// more for K/V that four times as many workgroups fetch, and 1.1 tiles to start and merge each workgroup.
+// D=64, causal unless said, us plain and KS: B=2 H=4 N=256 22.3 and 10.0; 8 heads N=1000 74.9 and 25.2; B=4 H=8
+// N=1000 78.2 and 59.6 (not causal 84.4 and 95.9); B=8 H=16 N=256 24.6 and 29.4; B=8 H=16 N=2048 570 and 725.
+static bool f32_key_split_pays(const fa_fwd_params& p) {
+  constexpr double kCus = 256;
+  const double heads = (double)p.batch * p.heads_q, tiles = (p.seqlen_k + 31) / 32;
+  auto mean_tiles = [&](int rows) {  // over the row blocks; a causal first block sees nk - nq + rows keys
+    if (!p.causal) return tiles;
+    return 0.5 * (tiles + std::min(tiles, std::max(1.0, (double)(p.seqlen_k - p.seqlen_q + rows) / 32)));
+  };
+  const double plain_wgs = heads * ((p.seqlen_q + 127) / 128), ks_wgs = heads * ((p.seqlen_q + 31) / 32);
+  const double plain = std::max(tiles, plain_wgs * mean_tiles(128) / kCus);
+  const double ks = std::max(1.1 * tiles / 4 + 1.1, ks_wgs / kCus * (1.1 * (mean_tiles(32) + 1.5) / 4 + 1.1));
+  return ks < plain;
+}
 
 fa_status run_fwd_f32(const fa_fwd_params& p, bool varlen, hipStream_t stream, const char** err) {
   TileArgs a = common_args(p);
@@ -289,17 +404,19 @@ fa_status run_fwd_f32(const fa_fwd_params& p, bool varlen, hipStream_t stream, c
     a.sqb = a.skb = a.svb = a.sob = a.slb = 0;  // rows are addressed by packed token index
   }
   if (a.nq <= 0 || p.batch <= 0) return FA_OK;
-  a.n_rowblk = (a.nq + 127) / 128;
+  const bool key_split = !varlen && p.head_dim <= 128 && f32_key_split_pays(p);
+  const int rpb = key_split ? 32 : 128;
+  a.n_rowblk = (a.nq + rpb - 1) / rpb;
   const int64_t total = (int64_t)p.batch * p.heads_q * a.n_rowblk;
   if (total > INT32_MAX) {
     *err = "grid too large";
     return FA_ERR_UNSUPPORTED;
   }
   a.total = (int32_t)total;
-  const hipError_t e = p.head_dim == 256 ? launch_f32<256>(a, stream)
-                       : p.head_dim == 128 ? launch_f32<128>(a, stream)
-                       : p.head_dim == 64 ? launch_f32<64>(a, stream)
-                                          : launch_f32<32>(a, stream);
+  const hipError_t e = p.head_dim == 256 ? launch_f32<256>(a, key_split, stream)
+                       : p.head_dim == 128 ? launch_f32<128>(a, key_split, stream)
+                       : p.head_dim == 64 ? launch_f32<64>(a, key_split, stream)
+                                          : launch_f32<32>(a, key_split, stream);
   return hip_status(e, err);
 }
 
