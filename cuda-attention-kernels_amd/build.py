@@ -1,5 +1,6 @@
 """Build ``fused_attn/libfused_attn_hip.so`` (and the measurement probe ``fused_attn/libfa_probe.so``)
-for gfx950 with hipcc.
+for gfx950 with hipcc, and the host-only ``fused_attn/libfused_attn_torch.so``, the native dispatcher
+kernels of the custom op, against the torch that runs this script.
 
     python cuda-attention-kernels_amd/build.py          # or __graft_entry__.build()
 
@@ -23,6 +24,8 @@ SOURCES = ["fa_prefill.hip", "fa_prefill_f32.hip", "fa_splitk.hip", "fa_generic.
 # the matrix-core ceiling probe bench.py times beside the prefill workload: a library of its own
 PROBE_SOURCES = ["fa_ceiling.hip"]
 PROBE_OUT = os.path.join(HERE, "fused_attn", "libfa_probe.so")
+TORCH_SOURCE = "fa_torch.cpp"
+TORCH_OUT = os.path.join(HERE, "fused_attn", "libfused_attn_torch.so")
 ARCH = os.environ.get("FUSED_ATTN_ARCH", "gfx950")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -54,9 +57,27 @@ def _run(cmd: list[str]) -> None:
         print(err, file=sys.stderr)
 
 
+def _torch_commands() -> list[list[str]]:
+    """Compile and link commands of the dispatcher library."""
+    import torch
+
+    root = os.path.dirname(os.path.abspath(torch.__file__))
+    inc, lib = os.path.join(root, "include"), os.path.join(root, "lib")
+    rocm = os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include")
+    obj = os.path.join(BUILD_DIR, "fa_torch.o")
+    compile_ = [HIPCC, "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+                f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-isystem", inc,
+                "-isystem", os.path.join(inc, "torch", "csrc", "api", "include"), "-isystem", rocm,
+                "-c", os.path.join(CSRC, TORCH_SOURCE), "-o", obj]
+    link = [HIPCC, "-shared", "-fPIC", obj, "-L", lib, "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-o",
+            TORCH_OUT + ".tmp"]
+    return [compile_, link]
+
+
 def build(verbose: bool = False) -> str:
     os.makedirs(BUILD_DIR, exist_ok=True)
-    cmds = []
+    torch_compile, torch_link = _torch_commands()
+    cmds = [torch_compile]
 
     def objects(sources):
         objs = []
@@ -69,6 +90,10 @@ def build(verbose: bool = False) -> str:
     libs = [(LIB_OUT, objects(SOURCES)), (PROBE_OUT, objects(PROBE_SOURCES))]
     with ThreadPoolExecutor(max_workers=len(cmds)) as ex:
         list(ex.map(_run, cmds))
+    _run(torch_link)
+    os.replace(TORCH_OUT + ".tmp", TORCH_OUT)
+    if verbose:
+        print(f"built {TORCH_OUT}")
     for out, objs in libs:
         tmp = out + ".tmp"
         _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp])

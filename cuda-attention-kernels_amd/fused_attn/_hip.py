@@ -18,6 +18,7 @@ import ctypes
 import math
 import os
 import threading
+import warnings
 from typing import Optional
 
 import torch
@@ -194,6 +195,46 @@ def library_loaded() -> bool:
         return True
     except RuntimeError:
         return False
+
+
+TORCH_LIB_NAME = "libfused_attn_torch.so"
+_native: Optional[ctypes.CDLL] = None
+_native_devices: set[int] = set()
+
+
+def load_native() -> None:
+    """Load the native dispatcher kernels of ``fused_attn::attention`` (csrc/fa_torch.cpp), if they are built for this
+    torch: they hand every call back to the Python kernels until ``_enable_native`` names its device."""
+    global _native
+    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), TORCH_LIB_NAME)
+    if _native is not None or torch.version.hip is None or not os.path.exists(path):
+        return
+    try:
+        torch.ops.load_library(path)
+        lib = ctypes.CDLL(path)
+    except OSError as e:  # built for another torch
+        warnings.warn(f"fused_attn: {path} does not load, calls take the slower Python path: {e}")
+        return
+    lib.fa_torch_bind.argtypes = [ctypes.c_void_p] * 5
+    lib.fa_torch_bind.restype = None
+    lib.fa_torch_enable.argtypes = [ctypes.c_int32]
+    lib.fa_torch_enable.restype = None
+    lib.fa_torch_route.argtypes = [ctypes.c_int32] + [ctypes.c_int64] * 6
+    lib.fa_torch_route.restype = ctypes.c_int64
+    _native = lib
+
+
+def _enable_native(index: int) -> None:
+    """Let the native kernels serve device ``index``, which ``device_supported`` has accepted."""
+    hip = load_library()
+    with _lock:
+        if _native is not None:
+            if not _native_devices:
+                _native.fa_torch_bind(*(ctypes.cast(f, ctypes.c_void_p) for f in (
+                    hip.fa_attention_fwd_workspace_bytes, hip.fa_attention_fwd_ws, hip.fa_splitk_workspace_bytes,
+                    hip.fa_attention_splitk, hip.fa_last_error)))
+            _native.fa_torch_enable(index)
+        _native_devices.add(index)
 
 
 _device_ok: dict[int, bool] = {}
@@ -417,6 +458,8 @@ def _require_gpu(*ts: torch.Tensor) -> None:
         raise RuntimeError(
             f"fused_attn HIP backend unavailable on {dev}: "
             + (_lib_error or "device is not a gfx950 GPU (set FUSED_ATTN_BACKEND=reference to run the unfused path)"))
+    if dev.index not in _native_devices:
+        _enable_native(dev.index)
 
 
 # ----------------------------------------------------------------------------------------------

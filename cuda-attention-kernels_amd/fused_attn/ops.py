@@ -138,6 +138,11 @@ def _attention_fake(q, k, v, causal=False, scale=None):
     return q.new_empty(q.shape)
 
 
+# GPU calls that need no preparation are launched by native dispatcher kernels; the function above stays the
+# kernel of all others, and the place that says what is accepted.
+_hip.load_native()
+
+
 def default_split_len(seqlen_q: int, seqlen_k: int, batch: int = 1, heads_kv: int = 1, group: int = 1) -> int:
     """Keys per split-K partition when the caller does not choose one.
 
