@@ -100,6 +100,7 @@ size_t fwd_workspace_bytes(const fa_fwd_params& p);
 // How run_fwd cuts a 16-bit call up: waves (of 32 queries) per workgroup, key splits per row block.
 struct FwdPlan {
   int nw, n_split;
+  bool short_tile;  // D=64 and D=32: 64-key tiles, three workgroups per CU
 };
 constexpr int kMaxFwdSplit = 32;
 FwdPlan plan_fwd(const fa_fwd_params& p, bool varlen, bool workspace);

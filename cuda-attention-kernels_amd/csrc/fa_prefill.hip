@@ -55,15 +55,15 @@ __device__ __forceinline__ void static_for(F&& f) {
 
 // a.n_split > 1 cuts a row block's key tiles over that many workgroups; each then writes an fp32
 // partial, and prefill_combine_kernel merges them (plan_fwd says when).
-template <int D, class E, int NW>
-__global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2)))
+// Keys per tile (BN): 64 at D=128, 32 at D=256, 128 at D <= 64: 16 KiB per K (or V) tile at D >= 64 and
+// 32 MFMAs per iteration; D=32 and D=16 keep 128 keys, whose scores already take 64 registers per lane.
+// At D=256 the fp32 output accumulator alone takes 128 registers per lane, so the kernel runs one wave per
+// SIMD there.  D=64 and D=32 also come with 64-key tiles, which leave registers and LDS for three
+// workgroups per CU in place of two (kFwdShortTile; plan_fwd says when).
+template <int D, class E, int NW, int BN>
+__global__ void __launch_bounds__(NW * 64)
+    __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : (D < 128 && BN == 64 ? 3 : 2))))
 attn_fwd_kernel(const TileArgs a) {
-  // 64-key tiles at D=128, 128-key tiles at D=64, 32-key tiles at D=256: 16 KiB per K (or V)
-  // tile and 32 MFMAs per iteration (measured: D=64 prefill 3% faster than with 64-key
-  // tiles).  D=32 and D=16 keep 128-key tiles: the scores of a tile already take 64 registers
-  // per lane.  At D=256 the fp32 output accumulator alone takes 128 registers per lane, so the
-  // kernel runs one wave per SIMD there.
-  constexpr int BN = D <= 64 ? 128 : (D == 256 ? 32 : 64);
   static_assert(NW == 4 || (NW == 8 && D != 256), "4 or 8 waves (two per SIMD) per workgroup");
   // V tiles are at least 32 columns wide, since O^T += V^T P^T works in 32-wide d blocks.  At
   // D=16 the upper 16 columns of a V row in LDS repeat the lower ones (the DMA reads each source
@@ -667,9 +667,12 @@ static hipError_t launch_prefill_combine(const CombineArgs& c, int64_t heads, hi
   return hipGetLastError();
 }
 
-template <int D, class E, int NW>
+constexpr int kFwdShortTile = 64;  // keys per tile of the three-workgroup form of D=64 and D=32
+constexpr int fwd_tile_keys(int d) { return d <= 64 ? 128 : (d == 256 ? 32 : 64); }
+
+template <int D, class E, int NW, int BN = fwd_tile_keys(D)>
 static hipError_t launch_fwd(const TileArgs& a, hipStream_t stream) {
-  hipLaunchKernelGGL((attn_fwd_kernel<D, E, NW>), dim3((unsigned)a.total), dim3(NW * 64), 0, stream, a);
+  hipLaunchKernelGGL((attn_fwd_kernel<D, E, NW, BN>), dim3((unsigned)a.total), dim3(NW * 64), 0, stream, a);
   return hipGetLastError();
 }
 
@@ -677,6 +680,9 @@ template <int D, class E>
 static hipError_t launch_fwd_plan(const TileArgs& a, const FwdPlan& plan, hipStream_t stream) {
   if constexpr (D == 128) {
     if (plan.nw == 8) return launch_fwd<D, E, 8>(a, stream);
+  }
+  if constexpr (D == 64 || D == 32) {
+    if (plan.short_tile) return launch_fwd<D, E, 4, kFwdShortTile>(a, stream);
   }
   return launch_fwd<D, E, 4>(a, stream);
 }
@@ -699,6 +705,14 @@ FwdPlan plan_fwd(const fa_fwd_params& p, bool varlen, bool workspace) {
   FwdPlan plan{};
   plan.nw = (d == 128 && nq >= (p.causal ? 4096 : 2048)) ? 8 : 4;
   plan.n_split = 1;
+  // D=64 and D=32 grids beyond two workgroups per CU take 64-key tiles and run three: the extra wave per
+  // SIMD hides more, and the last round is shorter.  Up to 512 workgroups the longer tile's iterations are
+  // the faster, and so they are at D=32 over more than 4096 keys.  GPU time, us, 128-key and 64-key tiles, D=64:
+  // B=8 H=16 N=577 28.9 and 25.9 (640 workgroups), B=32 87.6 and 74.6; causal Hq=32 B=8 N=700 40.0 and 35.6, B=4
+  // N=4096 323 and 312, B=1 N=8192 300 and 300, but N=1999 (512) 29.6 and 31.8.  D=32: B=32 H=16 N=577 64.6 and
+  // 56.4, causal Hq=32 B=4 N=4096 236 and 232, B=1 N=8192 207 and 215, N=1999 22.8 and 25.6.
+  plan.short_tile = (d == 64 || (d == 32 && nk <= 4096)) &&
+                    (int64_t)p.batch * p.heads_q * ((nq + 127) / 128) > 2 * kCus;
 
   // Key splits: a call whose row blocks leave compute units idle (few queries against many keys)
   // cuts each block's keys over several workgroups.  The estimate below, in microseconds, charges
@@ -709,7 +723,7 @@ FwdPlan plan_fwd(const fa_fwd_params& p, bool varlen, bool workspace) {
   // splits: 143 with 128-query blocks); 64 queries against 33000: 441 -> 68; 1000 queries against
   // 3000 (256 row blocks) stay unsplit at 52 (2 splits: 58).
   const int64_t heads = (int64_t)p.batch * p.heads_q;
-  const int bn = d <= 64 ? 128 : (d == 256 ? 32 : 64);
+  const int bn = fwd_tile_keys(d);
   if (varlen || !workspace || nk <= 0 || heads * ((nq + 127) / 128) > kCus) return plan;
   const double tiles = (nk + bn - 1) / bn;  // of the last (heaviest) row block
   // mean over the row blocks: a causal first block sees nk - nq + 128 keys
