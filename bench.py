@@ -339,7 +339,7 @@ def bench_decode(steps, warmup, only_128=False):
     kc, vc, ksp, vsp, bt, sl = fused_attn.paged_from_dense_fp8(k8, ks, v8, vs, 64,
                                                                generator=torch.Generator().manual_seed(0))
     for split in (128, None):
-        keys = split or fused_attn.ops.default_split_len(1, c["nk"], c["b"], c["hkv"], c["hq"] // c["hkv"])
+        keys = split or fused_attn.paged.default_paged_split_len(1, c["nk"], c["b"], c["hkv"], c["hq"] // c["hkv"], c["d"])
         fn = lambda: fused_attn.attention_paged(q, kc, vc, bt, sl, max_seqlen_k=c["nk"], split_len=keys,  # noqa: E731
                                                 k_scale=ksp, v_scale=vsp)
         err = _ref_err(fn()[:1], q[:1], kd0, vd0, False)
@@ -481,7 +481,7 @@ def bench_paged(k, v, steps, warmup, g, page_size=64, splits=(128, None), suffix
     q = torch.randn(c["b"], c["hq"], 1, c["d"], device="cuda", generator=g).bfloat16()
     res = {}
     for split in splits:
-        keys = split or fused_attn.ops.default_split_len(1, c["nk"], c["b"], c["hkv"], c["hq"] // c["hkv"])
+        keys = split or fused_attn.paged.default_paged_split_len(1, c["nk"], c["b"], c["hkv"], c["hq"] // c["hkv"], 2 * c["d"])
         keys = min(keys, max(64, (254 * page_size) // 64 * 64))  # as the op caps it for small pages
         fn = lambda: fused_attn.attention_paged(q, kc, vc, bt, sl, max_seqlen_k=c["nk"], split_len=keys)  # noqa: E731
         err = _batch0_err(fn(), q, k, v, False)  # the pool holds the dense K/V, shuffled into pages
