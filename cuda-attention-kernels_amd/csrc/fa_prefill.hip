@@ -53,14 +53,16 @@ __device__ __forceinline__ void static_for(F&& f) {
   }
 }
 
-// a.n_split > 1 cuts a row block's key tiles over that many workgroups; each then writes an fp32
-// partial, and prefill_combine_kernel merges them (plan_fwd says when).
+// SPLIT: a.n_split workgroups share a row block's key tiles; each writes an fp32 partial, and
+// prefill_combine_kernel merges them (plan_fwd says when).  A kernel of its own: with the split decided
+// at run time every call paid for it (GPU time, us, D=64 B=4 H=16 N=130 7.36 -> 7.60, D=128 B=1 Hq=20 Hkv=4
+// N=500 13.3 -> 13.7, D=128 not causal B=17 H=16 N=256 24.2 -> 24.9; 238 VGPRs in place of 229).
 // Keys per tile (BN): 64 at D=128, 32 at D=256, 128 at D <= 64: 16 KiB per K (or V) tile at D >= 64 and
 // 32 MFMAs per iteration; D=32 and D=16 keep 128 keys, whose scores already take 64 registers per lane.
 // At D=256 the fp32 output accumulator alone takes 128 registers per lane, so the kernel runs one wave per
 // SIMD there.  D=64 and D=32 also come with 64-key tiles, which leave registers and LDS for three
 // workgroups per CU in place of two (kFwdShortTile; plan_fwd says when).
-template <int D, class E, int NW, int BN>
+template <int D, class E, int NW, int BN, bool SPLIT>
 __global__ void __launch_bounds__(NW * 64)
     __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : (D < 128 && BN == 64 ? 3 : 2))))
 attn_fwd_kernel(const TileArgs a) {
@@ -110,9 +112,9 @@ attn_fwd_kernel(const TileArgs a) {
   PrefillItem it;
   if (!prefill_item<D>(a, it)) return;  // grid padding (uniform over the workgroup)
   const int b = it.b, hq = it.hq, kvh = it.kvh;
-  // a.n_rowblk counts (row block, key split) pairs, the splits of a row block side by side
-  const int rb = a.n_split > 1 ? it.rb / a.n_split : it.rb;
-  const int sp = a.n_split > 1 ? it.rb - rb * a.n_split : 0;
+  // SPLIT: a.n_rowblk counts (row block, key split) pairs, the splits of a row block side by side
+  const int rb = SPLIT ? it.rb / a.n_split : it.rb;
+  const int sp = SPLIT ? it.rb - rb * a.n_split : 0;
 
   int seq_q = a.nq, seq_k = a.nk;
   int64_t qtok0 = 0, ktok0 = 0;
@@ -133,7 +135,7 @@ attn_fwd_kernel(const TileArgs a) {
   int khi = seq_k;
   if (a.causal) khi = min(khi, min(r0 + NW * 32, seq_q) - 1 + offset + 1);
   int tile0 = 0;  // first tile of this workgroup's key range
-  if (a.n_split > 1) {
+  if constexpr (SPLIT) {
     const int per = ((khi > 0 ? (khi + BN - 1) / BN : 0) + a.n_split - 1) / a.n_split;
     tile0 = sp * per;
     khi = min(khi, (tile0 + per) * BN);
@@ -145,7 +147,7 @@ attn_fwd_kernel(const TileArgs a) {
   // Tile t of this workgroup's key range starts at key0(t); local_tiles(n) of the call's first n
   // tiles belong to it or to an earlier split.
   auto key0 = [&](int t) __attribute__((always_inline)) { return (tile0 + t) * BN; };
-  auto local_tiles = [&](int n) __attribute__((always_inline)) { return max(n - tile0, 0); };
+  auto local_tiles = [&](int n) __attribute__((always_inline)) { return SPLIT ? max(n - tile0, 0) : n; };
   const int n_tiles = local_tiles(khi > 0 ? (khi + BN - 1) / BN : 0);
   // Tiles [0, n_fast) hold only keys that every query of the workgroup sees.
   const int wg_mask_from = a.causal ? min(khi, r0 + offset + 1) : khi;
@@ -496,7 +498,7 @@ attn_fwd_kernel(const TileArgs a) {
   if (!wave_active) return;
   // each lane summed its 16 of the row's keys per tile (or holds the full sum, MFMA_ROWSUM)
   const float l_tot = MFMA_ROWSUM ? l_acc[0] : sum_xor32(l_run);
-  if (a.n_split > 1) {
+  if constexpr (SPLIT) {
     // fp32 partial of key split sp: O normalised by its own row sum (zeros for a row without keys
     // here) and (m, l), [S][B, Hq, Nq][D]
     const int64_t rows = (int64_t)a.kv_groups * a.group * seq_q;
@@ -670,19 +672,20 @@ static hipError_t launch_prefill_combine(const CombineArgs& c, int64_t heads, hi
 constexpr int kFwdShortTile = 64;  // keys per tile of the three-workgroup form of D=64 and D=32
 constexpr int fwd_tile_keys(int d) { return d <= 64 ? 128 : (d == 256 ? 32 : 64); }
 
-template <int D, class E, int NW, int BN = fwd_tile_keys(D)>
+template <int D, class E, int NW, bool SPLIT = false, int BN = fwd_tile_keys(D)>
 static hipError_t launch_fwd(const TileArgs& a, hipStream_t stream) {
-  hipLaunchKernelGGL((attn_fwd_kernel<D, E, NW, BN>), dim3((unsigned)a.total), dim3(NW * 64), 0, stream, a);
+  hipLaunchKernelGGL((attn_fwd_kernel<D, E, NW, BN, SPLIT>), dim3((unsigned)a.total), dim3(NW * 64), 0, stream, a);
   return hipGetLastError();
 }
 
 template <int D, class E>
 static hipError_t launch_fwd_plan(const TileArgs& a, const FwdPlan& plan, hipStream_t stream) {
   if constexpr (D == 128) {
-    if (plan.nw == 8) return launch_fwd<D, E, 8>(a, stream);
+    if (plan.nw == 8) return plan.n_split > 1 ? launch_fwd<D, E, 8, true>(a, stream) : launch_fwd<D, E, 8>(a, stream);
   }
+  if (plan.n_split > 1) return launch_fwd<D, E, 4, true>(a, stream);
   if constexpr (D == 64 || D == 32) {
-    if (plan.short_tile) return launch_fwd<D, E, 4, kFwdShortTile>(a, stream);
+    if (plan.short_tile) return launch_fwd<D, E, 4, false, kFwdShortTile>(a, stream);
   }
   return launch_fwd<D, E, 4>(a, stream);
 }
