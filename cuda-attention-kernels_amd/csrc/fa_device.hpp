@@ -249,7 +249,7 @@ __device__ __forceinline__ void st8(void* p, const u32x2& v) { *reinterpret_cast
 // Physical workgroup id -> logical id such that each XCD (8 per MI355X, each
 // with its own L2) receives a contiguous range of logical ids.  Workgroups are
 // dispatched round-robin over XCDs, so id p runs on XCD p % 8.
-__device__ __forceinline__ int xcd_remap(int pid, int total) {
+__host__ __device__ inline int xcd_remap(int pid, int total) {
   constexpr int kXcds = 8;
   const int q = total / kXcds, r = total % kXcds;
   const int xcd = pid % kXcds, slot = pid / kXcds;

@@ -53,6 +53,7 @@ struct TileArgs {
   int32_t o16;  // prefill: O base and strides allow 16-byte stores
   // dense prefill: pair heavy and light workgroups on a CU; deal the workgroups to the XCDs
   int32_t fold, deal;
+  int32_t share;  // dense causal prefill: q-heads of one XCD, 0 for one order over all heads
   int32_t batch, n_items;  // paged split-K: sequences, and batch * hkv * n_chunk
   int32_t u_heads, u_items;  // dense prefill schedule: q-heads per scheduling unit, and times n_rowblk
 };

@@ -801,14 +801,8 @@ fa_status run_fwd(const fa_fwd_params& p, bool varlen, hipStream_t stream, const
   }
   a.total = (int32_t)total;
   a.kv_groups = (int32_t)kv_groups;
-  // a unit never holds more than the (batch, q-head) pairs there are, which keeps u_items <= total
-  const int64_t bh = kv_groups * a.group;
-  a.deal = !varlen && prefill_deal(p.causal != 0, bh);
-  a.u_heads = (int32_t)(a.deal ? bh : std::min<int64_t>(prefill_unit_heads(a.nk, p.head_dim, a.group),
-                                                        prefill_unit_cap(p.causal != 0, bh, a.group)));
-  a.u_items = a.u_heads * a.n_rowblk;
   a.n_split = plan.n_split;
-  a.fold = (!varlen && p.causal && plan.nw == 4 && p.head_dim <= 128 && total > 256 && total <= 512) ? 1 : 0;
+  if (!varlen) prefill_schedule(a, p.head_dim, plan.nw);
   hipError_t e = hipErrorInvalidValue;
   const bool bf = p.dtype == FA_DTYPE_BF16;
   switch (p.head_dim) {

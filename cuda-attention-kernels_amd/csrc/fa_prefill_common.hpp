@@ -2,6 +2,8 @@
 // (fa_prefill.hip), kept apart from the kernel body.
 #pragma once
 
+#include <algorithm>
+
 #include "fa_device.hpp"
 #include "fa_internal.hpp"
 
@@ -18,7 +20,7 @@ struct PrefillItem {
 //
 // Dense: scheduling units are the q-heads of as many kv-heads as keep about unit_bytes of
 // K/V (prefill_unit_bytes; one XCD's L2 is 4 MB).  Units follow each other in logical order, and
-// xcd_remap hands each XCD a contiguous range of logical indices, so an XCD works through one
+// each XCD gets a contiguous range of it, so an XCD works through one
 // or two units at a time and re-reads K/V from its L2.  Inside a unit the query blocks go by
 // rank, heaviest causal blocks first, all heads of the unit at each rank, which keeps the
 // XCD's CUs evenly loaded to the end.
@@ -40,29 +42,84 @@ struct PrefillItem {
 // cost 2-8% (MHA D=64 N=4096: fewer heads to spread over the XCD's CUs), so those keep 4 MB.
 inline int64_t prefill_unit_bytes(int head_dim) { return int64_t{head_dim == 128 ? 2 : 4} << 20; }
 
-// q-heads per dense scheduling unit: the q-heads of as many whole kv-heads as fit
-// prefill_unit_bytes.  The host computes it once per launch (TileArgs::u_heads).
+// The q-heads of as many whole kv-heads as fit prefill_unit_bytes: the most a dense scheduling unit holds.
 inline int prefill_unit_heads(int nk, int head_dim, int group) {
   const int64_t kv_head_bytes = (int64_t)(nk > 1 ? nk : 1) * head_dim * 2 * 2;
   const int64_t kv_heads = prefill_unit_bytes(head_dim) / kv_head_bytes;
   return (int)(kv_heads > 1 ? kv_heads : 1) * group;
 }
 
-// Causal: a unit must not be cut by an XCD boundary, since its first half holds the heavier ranks
-// (the prompt of one request, Hq=32 Hkv=8 N=1999: an 8-head unit put ranks 16-9 on one XCD and 8-1
-// on the next, 1.47 times the mean), so a unit takes at most an XCD's share of the heads, and a call
-// with fewer than 32 heads that do not divide evenly is dealt to the XCDs rank by rank.
-inline bool prefill_deal(bool causal, int64_t heads) { return causal && heads < 32 && heads % 8 != 0; }
-inline int64_t prefill_unit_cap(bool causal, int64_t heads, int group) {
-  const int64_t share = heads / 8;
-  if (!causal || share < 1) return heads;
-  return share > group ? share / group * group : share;
+// Causal: an XCD's range must start with its heaviest blocks and end with its lightest.  A unit cut by a
+// range's end leaves ranks 16-9 on one XCD and 8-1 on the next (the prompt of one request, Hq=32 Hkv=8
+// N=1999, 8-head units: 1.47 times the mean load), or the heaviest blocks of the next unit to an XCD's last
+// round (D=128 B=7 Hq=16 Hkv=4 N=600, 24-head units 29.4 us, 12-head units 35.3, an XCD's own 14 heads 26.2).
+// Where the heads divide by the 8 XCDs each XCD therefore takes its share of them in units of its own: as few
+// as keep to prefill_unit_heads, of nearly equal size.  B=9 Hq=8 Hkv=1 N=1100 46.1 -> 38.7 us, B=3 Hq=16
+// Hkv=4 N=1500 50.0 -> 41.0, B=8 Hq=32 Hkv=8 N=700 64.1 -> 60.2.
+// q-heads of one XCD, 0 where the XCDs' ranges do not hold whole heads (or need not: without the causal mask)
+inline int prefill_share(bool causal, int64_t heads) { return causal && heads % 8 == 0 ? (int)(heads / 8) : 0; }
+// Heads that do not divide are dealt to the XCDs rank by rank where that beats one order over all heads: grids
+// of more than one workgroup per CU, with fewer than 32 heads or D <= 64 (D=64 B=7 Hq=12 N=1500 49.1 -> 38.6
+// us; 25 heads N=1300 D=128 35.5 -> 27.5).  Dealt, every XCD reads every K/V: with more heads at D >= 128 that
+// can cost what the balance gains (B=9 Hq=12 Hkv=4 N=1500, D=128 94.8 -> 86.6, D=256 176 -> 187).
+inline bool prefill_deal(bool causal, int64_t heads, int64_t total, int head_dim) {
+  return causal && heads % 8 != 0 && total > 256 && (heads < 32 || head_dim <= 64);
+}
+inline int64_t prefill_units(bool causal, int64_t heads, int group, int nk, int head_dim) {
+  const int64_t most = std::min<int64_t>(prefill_unit_heads(nk, head_dim, group), heads);
+  const int64_t share = prefill_share(causal, heads);
+  if (share == 0) return most;
+  if (share <= most) return share;
+  const int64_t units = (share + most - 1) / most, even = (share + units - 1) / units;
+  return (even + group - 1) / group * group;  // whole kv-heads: at most `most`, itself a multiple of group
+}
+
+// The schedule fields of a dense call's arguments (kv_groups, group, nk, causal, n_rowblk and total are set;
+// nw: waves per workgroup).
+inline void prefill_schedule(TileArgs& a, int head_dim, int nw) {
+  const bool causal = a.causal != 0;
+  const int64_t heads = (int64_t)a.kv_groups * a.group;
+  a.deal = prefill_deal(causal, heads, a.total, head_dim);
+  a.share = prefill_share(causal, heads);
+  // at most `heads`, so that u_items <= total
+  a.u_heads = (int32_t)(a.deal ? heads : prefill_units(causal, heads, a.group, a.nk, head_dim));
+  a.u_items = a.u_heads * a.n_rowblk;
+  // (in one order over all heads a range starts anywhere in a unit: reversed, B=3 Hq=12 Hkv=4 N=1000 D=128
+  // 26.8 -> 29.8 us)
+  a.fold = causal && (a.deal || a.share > 0) && nw == 4 && head_dim <= 128 && a.total > 256 && a.total <= 512;
+}
+
+struct PrefillOrder {
+  uint32_t rank, head;  // head: (batch, q-head) pair
+};
+
+// Workgroup -> rank and head of a dense call.  Every quantity is non-negative: unsigned division needs no
+// sign fix-ups, and all waves of the workgroup run this scalar code before their first DMA.
+__host__ __device__ inline PrefillOrder prefill_dense_order(const TileArgs& a, uint32_t bid) {
+  constexpr uint32_t kXcds = 8;
+  // a.fold: the grid fits the GPU at two workgroups per CU.  The dispatcher gives each of an XCD's 32
+  // CUs one workgroup and then a second, so the first 32 are taken in reverse: the CU with the heaviest
+  // of them gets the lightest of the rest (in order, the heaviest would get the heaviest again).
+  // With units cut to an XCD's share, Hq=32 Hkv=8 N=1999 causal D=128: 54.5 -> 45.6 us; 16 heads,
+  // N=4000: 97.8 -> 77.0.
+  uint32_t slot = bid / kXcds;
+  if (a.fold && slot < 32) slot = 31 - slot;
+  const uint32_t xcd = bid % kXcds, pid = slot * kXcds + xcd;
+  // the XCD's own heads (prefill_share), or one order over all heads: dealt to the XCDs one by one
+  // (a.deal), or a contiguous range each
+  const uint32_t heads = a.share > 0 ? (uint32_t)a.share : (uint32_t)a.kv_groups * (uint32_t)a.group;
+  const uint32_t first = xcd * (uint32_t)a.share;
+  const uint32_t logical = a.share > 0 ? slot : a.deal ? pid : (uint32_t)xcd_remap((int)pid, a.total);
+  const uint32_t unit = logical / (uint32_t)a.u_items;
+  const uint32_t within = logical - unit * (uint32_t)a.u_items;
+  const uint32_t left = heads - unit * (uint32_t)a.u_heads;
+  const uint32_t unit_size = left < (uint32_t)a.u_heads ? left : (uint32_t)a.u_heads;
+  const uint32_t rank = within / unit_size;
+  return {rank, first + unit * (uint32_t)a.u_heads + (within - rank * unit_size)};
 }
 
 template <int D>
 __device__ __forceinline__ bool prefill_item(const TileArgs& a, PrefillItem& it) {
-  // Every quantity here is non-negative: unsigned division needs no sign fix-ups, and all
-  // waves of the workgroup run this scalar code before their first DMA.
   constexpr uint32_t kXcds = 8;
   const uint32_t group = (uint32_t)a.group, bid = blockIdx.x;
   uint32_t mrev, item;
@@ -76,22 +133,9 @@ __device__ __forceinline__ bool prefill_item(const TileArgs& a, PrefillItem& it)
     if (kvg >= (uint32_t)a.kv_groups) return false;
     item = kvg * group + (j - jg * group);
   } else {
-    const uint32_t nbh = (uint32_t)a.kv_groups * group;  // (batch, q-head) pairs
-    // a.fold: the grid fits the GPU at two workgroups per CU.  The dispatcher gives each of an XCD's 32
-    // CUs one workgroup and then a second, so the first 32 are taken in reverse: the CU with the heaviest
-    // of them gets the lightest of the rest (in order, the heaviest would get the heaviest again).
-    // With units cut to an XCD's share, Hq=32 Hkv=8 N=1999 causal D=128: 54.5 -> 45.6 us; 16 heads,
-    // N=4000: 97.8 -> 77.0.
-    const uint32_t slot = bid / kXcds;
-    const uint32_t pid = a.fold && slot < 32 ? (31 - slot) * kXcds + bid % kXcds : bid;
-    // a.deal: one unit of all heads, its workgroups dealt to the XCDs one by one
-    const uint32_t logical = a.deal ? pid : (uint32_t)xcd_remap((int)pid, a.total);
-    const uint32_t unit_heads = (uint32_t)a.u_heads;  // prefill_unit_heads(nk, D, group)
-    const uint32_t unit = logical / (uint32_t)a.u_items;
-    const uint32_t within = logical - unit * (uint32_t)a.u_items;
-    const uint32_t unit_size = min(unit_heads, nbh - unit * unit_heads);
-    mrev = within / unit_size;
-    item = unit * unit_heads + (within - mrev * unit_size);
+    const PrefillOrder o = prefill_dense_order(a, bid);
+    mrev = o.rank;
+    item = o.head;
   }
   const uint32_t kvi = item / group;
   const uint32_t gi = item - kvi * group;
