@@ -40,10 +40,18 @@ int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 bool is_short_decode(int64_t b, int64_t hq, int64_t hkv, int64_t nq, int64_t nk, int64_t d) {
   const int64_t group = hq / hkv, heads = b * hq;
-  if (nq == 0 || group * nq > 32) return false;
-  if (group == 1) return nk >= 512 && heads <= 128 && nq <= 4 && d != 256;
-  if (heads > (d == 256 ? 256 : 512)) return nk >= 192;
-  return nk >= 512 && (d != 256 || heads > 64);
+  if (nq == 0 || group * nq > 32 || nq > 8) return false;
+  if (heads <= 64) return d != 256 && (group > 1 || nq <= 4) && nk >= (d == 64 ? 641 : 512);
+  const bool many = heads > (d == 256 ? 256 : 512);
+  if (group < 4) {
+    if (group == 1 || nq > 4) return false;
+    if (nq > 2) return nk >= 1600;
+    if (many) return nk >= (d == 64 ? 384 : 192);
+    return nk >= (d == 64 ? 1000 : d == 128 ? 768 : 512);
+  }
+  if (nq > 4) return nk >= (d == 64 ? 1600 : 1280);
+  if (many) return nk >= (d != 64 ? 192 : nq <= 2 ? 256 : 512);
+  return nk >= (d != 64 ? 512 : nq <= 2 ? 641 : 1000);
 }
 
 // Keys per split-K partition, or 0 for the prefill kernel.

@@ -10,7 +10,7 @@ ops.py:34-73, collapse into these two):
 
 * GPU tensors go to the HIP backend (``_hip``): MFMA FA2 prefill, or split-K
   flash-decoding for decode-shaped calls (at most 16 queries against at least
-  2048 keys, ops.py:36-37,63-66; grouped heads with few rows from 512 or 192).  If the HIP library cannot run on the device
+  2048 keys, ops.py:36-37,63-66; fewer for few rows, ``_is_short_decode``).  If the HIP library cannot run on the device
   the call raises; it never falls back silently.
 * CPU tensors, or ``FUSED_ATTN_BACKEND=reference``, use the unfused PyTorch
   path in ``reference.py``.
@@ -79,22 +79,35 @@ def _is_short_decode(q: torch.Tensor, k: torch.Tensor) -> bool:
 
     The prefill kernel gives every q-head a 128-row block and reads the K/V of a GQA group once per q-head;
     split-K takes the up to 32 (q-head, query) rows of a kv-head as one wave's rows and reads it once, but needs
-    a second launch.  GPU time, us, prefill kernel and split-K, D=128 bf16 Hq=32 Hkv=8, one query: 16 sequences
-    of 1000 keys 33.0 and 18.3, 40 of 256 keys 27.4 and 15.9, one of 700 keys 15.4 and 11.3; but one of 400 keys
-    at D=64 10.2 and 10.8, and 10 of 700 keys with 16 queries (64 rows) 23.7 and 31.2.  Without grouped heads
-    nothing is read twice: only a few heads, which leave the GPU idle, gain (32 heads, 700 keys 15.3 and 11.3).
-    At D=256 a small call stays with the prefill kernel (32 heads, 1200 keys 14.4 and 17.2)."""
+    a second launch, whose merge grows with the output rows.  It therefore needs the longer contexts, the more
+    queries there are and the fewer heads share a kv-head, and at D=64, where the prefill kernel's 128-key tiles
+    read half the bytes.  GPU time, us, prefill kernel and split-K, bf16: D=128 Hq=32 Hkv=8, one query, 16
+    sequences of 1000 keys 33.0 and 18.3, 40 of 256 keys 27.4 and 15.9; 8 queries, 32 of 192 keys 19.5 and 28.5;
+    D=64 with 64 heads 640 keys 10.1 and 11.1; Hq=16 Hkv=8, 8 queries, 32 of 1000 keys 31.7 and 42.2 (D=128), 22.7
+    and 28.9 (D=64).  Without grouped heads nothing is read twice: only a few heads, which leave the GPU idle,
+    gain.  At D=256 a small call stays with the prefill kernel (32 heads, 1200 keys 14.4 and 17.2)."""
     if q.dim() != 4 or k.dim() != 4 or k.shape[1] == 0 or q.shape[1] % k.shape[1] != 0:
         return False
     b, hq, nq, d = q.shape
     nk, group, heads = k.shape[2], hq // k.shape[1], b * hq
-    if nq == 0 or group * nq > 32:
+    if nq == 0 or group * nq > 32 or nq > 8:
         return False
-    if group == 1:
-        return nk >= 512 and heads <= 128 and nq <= 4 and d != 256
-    if heads > (256 if d == 256 else 512):
-        return nk >= 192
-    return nk >= 512 and (d != 256 or heads > 64)
+    if heads <= 64:
+        return d != 256 and (group > 1 or nq <= 4) and nk >= (641 if d == 64 else 512)
+    many = heads > (256 if d == 256 else 512)
+    if group < 4:
+        if group == 1 or nq > 4:
+            return False
+        if nq > 2:
+            return nk >= 1600
+        if many:
+            return nk >= (384 if d == 64 else 192)
+        return nk >= (1000 if d == 64 else 768 if d == 128 else 512)
+    if nq > 4:
+        return nk >= (1600 if d == 64 else 1280)
+    if many:
+        return nk >= (192 if d != 64 else 256 if nq <= 2 else 512)
+    return nk >= (512 if d != 64 else 641 if nq <= 2 else 1000)
 
 
 def _hip_kernel_for(q: torch.Tensor, k: torch.Tensor) -> str:

@@ -11,8 +11,18 @@ from oracle import attention_oracle as orc
 CASES = [  # b, hq, hkv, nq, nk, d -> kernel family
     ((2, 8, 2, 1, 511, 128), "fwd"), ((2, 8, 2, 1, 512, 128), "splitk"), ((2, 8, 2, 8, 700, 64), "splitk"),
     ((2, 8, 2, 9, 700, 64), "fwd"), ((2, 8, 2, 1, 1000, 256), "fwd"), ((9, 8, 2, 1, 1000, 256), "splitk"),
-    ((17, 32, 8, 1, 191, 128), "fwd"), ((17, 32, 8, 3, 192, 128), "splitk"), ((16, 8, 8, 4, 600, 64), "splitk"),
+    ((17, 32, 8, 1, 191, 128), "fwd"), ((17, 32, 8, 3, 192, 128), "splitk"), ((16, 8, 8, 4, 600, 64), "fwd"),
     ((16, 8, 8, 5, 600, 64), "fwd"), ((17, 8, 8, 1, 600, 64), "fwd"),
+    # the context from which each of these is faster grows with the queries, at D=64 and where few heads share a
+    # kv-head (us: prefill kernel and split-K)
+    ((8, 8, 8, 4, 640, 64), "fwd"), ((8, 8, 8, 4, 641, 64), "splitk"), ((16, 8, 8, 1, 1280, 128), "fwd"),
+    ((2, 32, 8, 1, 640, 64), "fwd"),  # 10.1 and 11.1
+    ((32, 32, 8, 8, 384, 64), "fwd"),  # 19.1 and 31.9
+    ((16, 32, 8, 8, 640, 128), "fwd"), ((16, 32, 8, 8, 1280, 128), "splitk"),
+    ((32, 16, 8, 8, 1600, 128), "fwd"),  # 46.1 and 53.7
+    ((64, 16, 8, 4, 192, 64), "fwd"),  # 12.7 and 20.8
+    ((16, 16, 8, 8, 1000, 256), "fwd"),  # 35.0 and 40.5
+    ((32, 64, 8, 2, 255, 64), "fwd"), ((32, 64, 8, 2, 256, 64), "splitk"),
 ]
 
 
