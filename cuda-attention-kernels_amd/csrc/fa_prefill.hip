@@ -709,12 +709,14 @@ FwdPlan plan_fwd(const fa_fwd_params& p, bool varlen, bool workspace) {
   plan.nw = (d == 128 && nq >= (p.causal ? 4096 : 2048)) ? 8 : 4;
   plan.n_split = 1;
   // D=64 and D=32 grids beyond two workgroups per CU take 64-key tiles and run three: the extra wave per
-  // SIMD hides more, and the last round is shorter.  Up to 512 workgroups the longer tile's iterations are
-  // the faster, and so they are at D=32 over more than 4096 keys.  GPU time, us, 128-key and 64-key tiles, D=64:
-  // B=8 H=16 N=577 28.9 and 25.9 (640 workgroups), B=32 87.6 and 74.6; causal Hq=32 B=8 N=700 40.0 and 35.6, B=4
-  // N=4096 323 and 312, B=1 N=8192 300 and 300, but N=1999 (512) 29.6 and 31.8.  D=32: B=32 H=16 N=577 64.6 and
-  // 56.4, causal Hq=32 B=4 N=4096 236 and 232, B=1 N=8192 207 and 215, N=1999 22.8 and 25.6.
-  plan.short_tile = (d == 64 || (d == 32 && nk <= 4096)) &&
+  // SIMD hides more, and the last round is shorter.  Up to 512 workgroups, and over more than 4096 keys, the
+  // longer tile's iterations are the faster.  GPU time, us, 128-key and 64-key tiles, D=64: B=8 H=16 N=577 28.9 and
+  // 25.9 (640 workgroups), B=32 87.6 and 74.6; causal Hq=32 B=8 N=700 40.0 and 35.6, B=4 N=4096 323 and 312, but N=1999
+  // (512) 29.6 and 31.8, H=16 N=6000 89.3 and 93.2, B=4 H=8 N=7000 215 and 237.  D=32: B=32 H=16 N=577 64.6 and 56.4,
+  // causal Hq=32 B=4 N=4096 236 and 232, B=1 N=8192 207 and 215, N=1999 22.8 and 25.6.  A varlen grid is laid out for
+  // its longest sequence and holds fewer workgroups than it counts: it keeps the longer tile (4 sequences up to
+  // 1500 tokens, 16 heads, D=64: 28.6 and 37.6).
+  plan.short_tile = !varlen && (d == 64 || d == 32) && nk <= 4096 &&
                     (int64_t)p.batch * p.heads_q * ((nq + 127) / 128) > 2 * kCus;
 
   // Key splits: a call whose row blocks leave compute units idle (few queries against many keys)
