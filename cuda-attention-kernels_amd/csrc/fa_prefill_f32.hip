@@ -73,10 +73,13 @@ attn_fwd_f32_kernel(const TileArgs a) {
 
   // ---- work item: (batch or sequence, q-head, 128-query block), rank-major ---------------
   // All (batch, q-head) pairs at one rank run together (heaviest causal blocks first), the
-  // q-heads of one kv-head side by side; xcd_remap gives each XCD a contiguous range.  Causal ranks
-  // are dealt to the XCDs instead: a contiguous range gave the first XCD all the heaviest.
+  // q-heads of one kv-head side by side; xcd_remap gives each XCD a contiguous range.  The ranks of a
+  // dense causal call are dealt to the XCDs instead: a contiguous range gave the first XCD all the heaviest
+  // (us, B=4 H=16 N=1024 D=32 / 64 / 128 / 256: 79 / 141 / 266 / 650 -> 57 / 104 / 190 / 354).  A varlen grid's
+  // heaviest ranks are mostly empty, and dealing spreads a sequence's K/V over all XCDs: 4 sequences up to
+  // 1500 tokens, 16 heads, D=64: 177 us in order and 197 dealt.
   const int nbh = a.total / a.n_rowblk;
-  const int logical = a.causal ? (int)blockIdx.x : xcd_remap((int)blockIdx.x, a.total);
+  const int logical = a.causal && !a.varlen ? (int)blockIdx.x : xcd_remap((int)blockIdx.x, a.total);
   const int mrev = logical / nbh;
   const int item = logical % nbh;
   const int hq = item % a.hq;
