@@ -115,6 +115,7 @@ attn_splitk_kernel(const TileArgs a) {
 
   // ---- work item: (batch, kv-head, chunk of ppw partitions, row block) -------------
   int rb, chunk, kvh, b;
+  bool idle = false;  // grid padding: exits below, with the workgroups past a sequence's end
   if constexpr (PAGED) {
     // Sequences differ in length, so the items are dealt to the XCDs one by one (a contiguous range
     // each, as below, gives an XCD whole sequences, and the one with the longest runs on alone), chunk
@@ -126,7 +127,8 @@ attn_splitk_kernel(const TileArgs a) {
     const int xcd = (int)blockIdx.x % 8, slot = (int)blockIdx.x / 8;
     rb = slot % a.n_rowblk;
     int item = (slot / a.n_rowblk) * 8 + xcd;
-    if (item >= a.n_items) return;  // padding: uniform over the workgroup
+    idle = item >= a.n_items;
+    item = idle ? 0 : item;
     kvh = item % a.hkv;
     item /= a.hkv;
     b = item % a.batch;
@@ -147,25 +149,10 @@ attn_splitk_kernel(const TileArgs a) {
   if constexpr (PAGED) seq_k = min(max(__builtin_amdgcn_readfirstlane(a.seqlens_k[b]), 0), a.nk);
   const int R = a.group * seq_q;  // rows: (q-head in group, query)
   const int r0 = rb * NW * 32;    // < R: the grid has ceil(R / (NW * 32)) row blocks
-  const int offset = seq_k - seq_q;  // bottom-right causal alignment (reference.py:24-33)
 
   const int part0 = chunk * a.ppw;
-  int part_end = min(part0 + a.ppw, a.n_split);
+  const int part_end = min(part0 + a.ppw, a.n_split);
   const int klo = part0 * a.split_len;
-  if constexpr (PAGED) {
-    // partitions past this sequence's end are neither written here nor read by the merge
-    if (klo >= seq_k) return;  // uniform over the workgroup
-    part_end = min(part_end, (seq_k - 1) / a.split_len + 1);
-  }
-  int khi = min(seq_k, part_end * a.split_len);
-  if (a.causal) {
-    // last query of the block (rows wrap around the queries once per q-head)
-    const int re = min(r0 + NW * 32, R);
-    const int qmax = (re - r0 >= seq_q || (r0 % seq_q) > ((re - 1) % seq_q)) ? seq_q - 1 : (re - 1) % seq_q;
-    khi = min(khi, qmax + offset + 1);
-  }
-  const int n_tiles = khi > klo ? (khi - klo + BN - 1) / BN : 0;
-  const int tiles_per_part = a.split_len / BN;  // split_len is a multiple of 64 (C ABI)
 
   // ---- lane roles ------------------------------------------------------------------
   const int tid = (int)threadIdx.x;
@@ -178,22 +165,39 @@ attn_splitk_kernel(const TileArgs a) {
   const bool wave_active = wr0 < R;
   const int hq = kvh * a.group + (row_ok ? row / seq_q : 0);
   const int qi = row_ok ? row % seq_q : 0;
-  // Keys visible to every row of the wave need no element-wise mask; keys at or
-  // beyond wave_khi are visible to no row of the wave.
-  int wave_khi = khi, mask_from = khi;
-  if (a.causal && wave_active) {
-    const int we = min(wr0 + 32, R);
-    int qlo, qhi;
-    if (we - wr0 >= seq_q || (wr0 % seq_q) > ((we - 1) % seq_q)) {
-      qlo = 0;
-      qhi = seq_q - 1;
-    } else {
-      qlo = wr0 % seq_q;
-      qhi = (we - 1) % seq_q;
+
+  // The keys this workgroup and this wave see.  Paged: after the loads below, since it waits for the
+  // sequence's length; a dense call has it ready and needs no such wait (there, late, it cost up to 3%).
+  const int tiles_per_part = a.split_len / BN;  // split_len is a multiple of 64 (C ABI)
+  int offset, khi, n_tiles, wave_khi, mask_from;
+  auto visible_keys = [&]() __attribute__((always_inline)) {
+    offset = seq_k - seq_q;  // bottom-right causal alignment (reference.py:24-33)
+    khi = min(seq_k, part_end * a.split_len);
+    if (a.causal) {
+      // last query of the block (rows wrap around the queries once per q-head)
+      const int re = min(r0 + NW * 32, R);
+      const int qmax = (re - r0 >= seq_q || (r0 % seq_q) > ((re - 1) % seq_q)) ? seq_q - 1 : (re - 1) % seq_q;
+      khi = min(khi, qmax + offset + 1);
     }
-    wave_khi = min(khi, qhi + offset + 1);
-    mask_from = min(khi, qlo + offset + 1);
-  }
+    n_tiles = khi > klo ? (khi - klo + BN - 1) / BN : 0;
+    // Keys visible to every row of the wave need no element-wise mask; keys at or
+    // beyond wave_khi are visible to no row of the wave.
+    wave_khi = mask_from = khi;
+    if (a.causal && wave_active) {
+      const int we = min(wr0 + 32, R);
+      int qlo, qhi;
+      if (we - wr0 >= seq_q || (wr0 % seq_q) > ((we - 1) % seq_q)) {
+        qlo = 0;
+        qhi = seq_q - 1;
+      } else {
+        qlo = wr0 % seq_q;
+        qhi = (we - 1) % seq_q;
+      }
+      wave_khi = min(khi, qhi + offset + 1);
+      mask_from = min(khi, qlo + offset + 1);
+    }
+  };
+  if constexpr (!PAGED) visible_keys();
 
   // K/V of this (batch, kv-head), read with buffer loads: a load past the
   // resource's byte limit returns zeros, which zero-fills the keys >= khi of the
@@ -235,7 +239,8 @@ attn_splitk_kernel(const TileArgs a) {
                         // which the K/V stream does not evict, so the first DMA waits little
   if constexpr (PAGED) {
     // bounded by the grid's largest length, not this sequence's, so that this load does
-    // not wait for seqlens_k[b] (both are in flight together); <= block_table_cols.
+    // not wait for seqlens_k[b] (both are in flight together, and Q with them: waiting for the
+    // length first cost every call 0.4 us); <= block_table_cols.
     // Issued before the Q loads: waiting for the entries then leaves Q in flight.
     first_slot = klo / a.page_size;
     const int kgrid = min(a.nk, part_end * a.split_len);
@@ -264,6 +269,12 @@ attn_splitk_kernel(const TileArgs a) {
   }
   // keep the Q loads ahead of the first K/V tiles' DMA: waiting for Q then leaves the tiles in flight
   __builtin_amdgcn_sched_barrier(0);
+
+  // paged: partitions past this sequence's end are neither written here nor read by the merge
+  if constexpr (PAGED) {
+    if (idle || klo >= seq_k) return;  // uniform over the workgroup
+    visible_keys();
+  }
 
   // page slot of key n >= 0: a multiply-high in place of a division by the page size
   auto slot_of = [&](int n) __attribute__((always_inline)) {
@@ -725,9 +736,12 @@ attn_splitk_kernel(const TileArgs a) {
     }
   }
 
-  // partitions past the visible keys (causal, or past the sequence end): empty
+  // partitions past the visible keys (causal; dense: or past the sequence end): empty
   // partials, m = -inf and l = 0, which the combine weighs by zero
-  for (int part = part0 + (n_tiles + tiles_per_part - 1) / tiles_per_part; part < part_end; ++part) emit_partial(part);
+  for (int part = part0 + (n_tiles + tiles_per_part - 1) / tiles_per_part; part < part_end; ++part) {
+    if (PAGED && part * a.split_len >= seq_k) break;
+    emit_partial(part);
+  }
 }
 
 // Log-sum-exp merge of split-K partials (triton_splitk.py:99-127), with each fp32 partial
@@ -737,7 +751,7 @@ attn_splitk_kernel(const TileArgs a) {
 // loads each (8 elements), so 256/(D/8) partials are read concurrently.  Each thread merges
 // its partials online (running max, rescaled sums), and the threads' (m, l, acc) triples
 // are merged through LDS at the end: one pass over the partials, no separate max pass.
-template <int D, class E, bool PART_MAJOR>
+template <int D, class E, bool PART_MAJOR, bool PAGED>
 __global__ void __launch_bounds__(256) splitk_combine_kernel(const CombineArgs c) {
   constexpr int TPS = D / 8;
   constexpr int SPB = 256 / TPS;
@@ -747,11 +761,13 @@ __global__ void __launch_bounds__(256) splitk_combine_kernel(const CombineArgs c
 
   const int64_t row = blockIdx.x;  // (b, hq, qi) flattened
   const int S = c.n_split;
-  int live = S;  // paged: only the partitions below the sequence's end were written
-  if (c.seqlens_k != nullptr) {
-    const int n = min(max(c.seqlens_k[(uint32_t)row / ((uint32_t)c.hq * (uint32_t)c.nq)], 0), c.nk);
-    live = n > 0 ? (n - 1) / c.split_len + 1 : 0;
-  }
+  // paged: only the partitions that start below the sequence's end were written
+  int end = 0;
+  if constexpr (PAGED) end = min(c.seqlens_k[(uint32_t)row / ((uint32_t)c.hq * (uint32_t)c.nq)], c.nk);
+  auto written = [&](int s) __attribute__((always_inline)) {
+    if constexpr (!PAGED) return s < S;
+    return s < S && (int)((uint32_t)s * (uint32_t)c.split_len) < end;  // (past S the product may wrap)
+  };
   // row-major partials: S consecutive rows; partition-major: one row of each of S blocks of
   // R = G * Nq rows (the grid has fewer than 2^31 rows: 32-bit index arithmetic)
   int64_t base = row * S, pstride = 1;
@@ -778,13 +794,13 @@ __global__ void __launch_bounds__(256) splitk_combine_kernel(const CombineArgs c
   constexpr int CH = 8;
   float m = NEG_INF, l = 0.f;
   f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-  for (int s0 = sg; s0 < live; s0 += CH * SPB) {
+  for (int s0 = sg; written(s0); s0 += CH * SPB) {
     f32x2 st[CH];
     f32x4 pv0[CH], pv1[CH];
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
       const int s = s0 + u * SPB;
-      if (s < live) {
+      if (written(s)) {
         st[u] = __builtin_bit_cast(f32x2, ld8(ml + 2 * s * pstride));
         pv0[u] = __builtin_bit_cast(f32x4, ld16(op + s * pstride * D + 8 * dq));
         pv1[u] = __builtin_bit_cast(f32x4, ld16(op + s * pstride * D + 8 * dq + 4));
@@ -859,10 +875,11 @@ static hipError_t launch_splitk(const TileArgs& a, hipStream_t stream) {
 template <int D, class E>
 static hipError_t launch_combine(const CombineArgs& c, int64_t rows, hipStream_t stream) {
   // the layout is a template argument: with a runtime stride the row-major merge ran 30-45% slower
-  if (c.part_major) {
-    hipLaunchKernelGGL((splitk_combine_kernel<D, E, true>), dim3((unsigned)rows), dim3(256), 0, stream, c);
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3(256), 0, stream, c); };
+  if (c.seqlens_k != nullptr) {
+    c.part_major ? launch(splitk_combine_kernel<D, E, true, true>) : launch(splitk_combine_kernel<D, E, false, true>);
   } else {
-    hipLaunchKernelGGL((splitk_combine_kernel<D, E, false>), dim3((unsigned)rows), dim3(256), 0, stream, c);
+    c.part_major ? launch(splitk_combine_kernel<D, E, true, false>) : launch(splitk_combine_kernel<D, E, false, false>);
   }
   return hipGetLastError();
 }
