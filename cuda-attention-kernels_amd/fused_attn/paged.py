@@ -33,7 +33,7 @@ import torch
 
 from . import _hip
 from .fp8 import FP8_DTYPE, QBLOCK, dequantize_kv_fp8
-from .ops import _pick_backend
+from .ops import _pick_backend, default_split_len
 from .reference import attention_reference, lse_reference
 
 
@@ -66,20 +66,26 @@ def default_paged_split_len(seqlen_q: int, max_seqlen_k: int, batch: int, heads_
 
     The grid is laid out for the longest sequence and the workgroups past a shorter one's end exit at
     once, so a ragged batch fills about half of it: it takes more, shorter partitions than a dense cache
-    (``ops.default_split_len``) to keep the GPU busy to the end.  The longest power of two (other lengths
-    measured up to 15% slower) with 2304 workgroups at 256-byte rows (D=128 in 16 bits; twice as many at
-    half the bytes), 128 to 4096; a batch too small for that takes 512 or shorter, with 1000 workgroups.
+    to keep the GPU busy to the end.  The longest power of two (other lengths measured up to 15% slower)
+    with 2304 workgroups at 256-byte rows (D=128 in 16 bits; half as many at twice the bytes), 512 to 4096; a
+    batch too small for that takes 128 or longer, with 1000 workgroups.
     D=128 bf16 Hkv=8, ragged, us at this length and at the dense policy's: 48 sequences up to 8192 keys
     132 (1024) and 150 (1408); 100 up to 2000, 81 (512) and 87 (704); 16 up to 4096 with Hkv=4, 25 (256)
-    and 31 (128); D=64, 48 up to 8192, 81 (512) and 112 (1408).
+    and 31 (128).
+
+    Rows of fewer than 256 bytes (D=64, FP8 at D=64 and D=128) take the dense policy: a short partition is
+    then half a partial's traffic, and what shorter ones gain for some ragged batches they lose for others
+    and for equal lengths (D=64 bf16 Hkv=8, 8 queries, 48 sequences of 8192 keys: 188 us at 512 and 164 at
+    1408; FP8 D=64, 16 queries, 24 sequences of 4000: 1.6 times at 128 of what it takes at 384).
     """
+    if row_bytes < 256:
+        return default_split_len(seqlen_q, max_seqlen_k, batch, heads_kv, group)
     rows = group * seqlen_q
     items = max(1, batch * heads_kv * -(-rows // 128))
-    scale = 256 / row_bytes
     keys = 4096
-    while keys > 512 and items * -(-max_seqlen_k // keys) < 2304 * scale:
+    while keys > 512 and items * -(-max_seqlen_k // keys) < 2304 * 256 / row_bytes:
         keys //= 2
-    while keys > 128 and items * -(-max_seqlen_k // keys) < 1000 * max(scale, 1.0):
+    while keys > 128 and items * -(-max_seqlen_k // keys) < 1000:
         keys //= 2
     return keys
 

@@ -59,9 +59,33 @@ def test_fp8_two_partitions_per_workgroup():
         assert max_err(out[i:i + 1], one.float().cpu()) <= TOL[torch.bfloat16]
 
 
-@pytest.mark.parametrize("row_bytes", [64, 128, 256, 512])
+@pytest.mark.parametrize("row_bytes", [256, 512])
 @pytest.mark.parametrize("n", [0, 1, 600, 8192, 1 << 20])
-@pytest.mark.parametrize("b,hkv,group,nq", [(1, 1, 1, 1), (48, 8, 4, 1), (300, 32, 8, 16)])
+@pytest.mark.parametrize("b,hkv,group,nq", [(1, 1, 1, 1), (16, 4, 4, 1), (48, 8, 4, 1), (100, 8, 4, 4), (300, 32, 8, 16)])
 def test_default_partitions(b, hkv, group, nq, n, row_bytes):
+    """The longest power of two whose grid reaches its target: 2304 workgroups (by 256-byte rows) down to 512 keys,
+    1000 below."""
     keys = default_paged_split_len(nq, n, b, hkv, group, row_bytes)
-    assert keys in (128, 256, 512, 1024, 2048, 4096)
+    large = 2304 * 256 // row_bytes
+
+    def workgroups(length):
+        return b * hkv * -(-group * nq // 128) * -(-n // length)
+
+    assert 128 <= keys <= 4096 and keys & (keys - 1) == 0
+    assert keys == 128 or workgroups(keys) >= (large if keys > 512 else 1000)
+    assert keys == 4096 or workgroups(2 * keys) < (large if keys >= 512 else 1000)
+
+
+@pytest.mark.parametrize("args,keys", [
+    ((1, 8192, 48, 8, 4, 256), 1024), ((1, 2000, 100, 8, 4, 256), 512), ((1, 4096, 16, 4, 4, 256), 256),
+    ((1, 2000, 100, 8, 4, 512), 1024),
+    # rows of fewer than 256 bytes: the dense policy
+    ((8, 8192, 48, 8, 4, 128), 1408), ((16, 4000, 24, 8, 8, 64), 384), ((1, 3000, 4, 32, 4, 128), 192),
+])
+def test_default_partitions_as_measured(args, keys):
+    assert default_paged_split_len(*args) == keys
+
+
+def test_default_partitions_of_a_malformed_head_dim():
+    """A head dim of 0 reaches the checks of the call itself."""
+    assert default_paged_split_len(1, 1000, 2, 2, 4, 0) == 128
