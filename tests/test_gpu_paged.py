@@ -9,10 +9,17 @@ import pytest
 import torch
 
 import fused_attn
+from fused_attn.paged import default_paged_split_len
 from helpers import TOL, announce, max_err, randn
 from oracle import attention_oracle as orc
 
 pytestmark = pytest.mark.gpu
+
+
+def _default(nq, n, b, hkv, group, d, page, itemsize=2):
+    """The partition a call without split_len takes: the policy's, within 256 pages."""
+    keys = default_paged_split_len(nq, n, b, hkv, group, d * itemsize)
+    return min(keys, max(64, 254 * page // 64 * 64))
 
 
 def _dense_and_paged(b, hq, hkv, nq, n, d, page, dtype, lens=None, seed=0, extra=3):
@@ -47,9 +54,9 @@ def test_paged_is_bit_identical_to_dense_splitk(split_len, nq, causal):
     """Equal lengths: the paged kernel equals the dense split-K kernel bit for bit."""
     announce(f"paged == dense split_len={split_len} nq={nq} causal={causal}")
     q, k, v, kc, vc, bt, sl = _dense_and_paged(3, 16, 4, nq, 777, 128, 64, torch.bfloat16)
-    sk = split_len or fused_attn.ops.default_split_len(nq, 777, 3, 4, 4)
+    sk = split_len or _default(nq, 777, 3, 4, 4, 128, 64)
     dense = fused_attn.attention_splitk(q, k, v, causal=causal, split_len=sk)
-    paged = fused_attn.attention_paged(q, kc, vc, bt, sl, causal=causal, split_len=sk)
+    paged = fused_attn.attention_paged(q, kc, vc, bt, sl, causal=causal, split_len=split_len)
     assert torch.equal(dense, paged)
 
 
@@ -62,9 +69,9 @@ def test_paged_small_pages_bit_identical_to_dense_splitk(page, d, split_len, nq,
     and the result still equals the dense split-K kernel bit for bit."""
     announce(f"paged small pages == dense page={page} d={d} split_len={split_len} nq={nq} causal={causal}")
     q, k, v, kc, vc, bt, sl = _dense_and_paged(2, 8, 2, nq, 700, d, page, torch.bfloat16)
-    sk = split_len or fused_attn.ops.default_split_len(nq, 700, 2, 2, 4)
+    sk = split_len or _default(nq, 700, 2, 2, 4, d, page)
     dense = fused_attn.attention_splitk(q, k, v, causal=causal, split_len=sk)
-    paged = fused_attn.attention_paged(q, kc, vc, bt, sl, causal=causal, split_len=sk)
+    paged = fused_attn.attention_paged(q, kc, vc, bt, sl, causal=causal, split_len=split_len)
     assert torch.equal(dense, paged)
 
 
@@ -153,9 +160,9 @@ def test_paged_decode_cache_size():
     announce("paged decode 32x32x32768x128")
     q, k, v, kc, vc, bt, sl = _dense_and_paged(32, 32, 8, 1, 32768, 128, 64, torch.bfloat16, extra=0)
     for split_len in (128, None):
-        sk = split_len or fused_attn.ops.default_split_len(1, 32768, 32, 8, 4)
+        sk = split_len or _default(1, 32768, 32, 8, 4, 128, 64)
         dense = fused_attn.attention_splitk(q, k, v, split_len=sk)
-        paged = fused_attn.attention_paged(q, kc, vc, bt, sl, max_seqlen_k=32768, split_len=sk)
+        paged = fused_attn.attention_paged(q, kc, vc, bt, sl, max_seqlen_k=32768, split_len=split_len)
         assert torch.equal(dense, paged), sk
 
 

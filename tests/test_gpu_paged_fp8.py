@@ -11,6 +11,7 @@ import pytest
 import torch
 
 import fused_attn
+from fused_attn.paged import default_paged_split_len
 from helpers import FP8_TOL, announce, max_err, randn
 from oracle import attention_oracle as orc
 
@@ -60,10 +61,21 @@ def test_paged_fp8_is_bit_identical_to_dense_fp8(split_len, nq, causal):
     announce(f"paged fp8 == dense fp8 split_len={split_len} nq={nq} causal={causal}")
     q, (k8, ks, v8, vs), (kc, vc, ksp, vsp, bt, sl) = _fp8_dense_and_paged(3, 16, 4, nq, 777, 128, 128,
                                                                            torch.bfloat16)
-    sk = split_len or fused_attn.ops.default_split_len(nq, 777, 3, 4, 4)
+    sk = split_len or default_paged_split_len(nq, 777, 3, 4, 4, 128)
     dense = fused_attn.attention_fp8(q, k8, ks, v8, vs, causal=causal, split_len=sk)
-    paged = fused_attn.attention_paged(q, kc, vc, bt, sl, causal=causal, split_len=sk, k_scale=ksp, v_scale=vsp)
+    paged = fused_attn.attention_paged(q, kc, vc, bt, sl, causal=causal, split_len=split_len, k_scale=ksp, v_scale=vsp)
     assert torch.equal(dense, paged)
+
+
+@pytest.mark.parametrize("d,keys", [(64, 128), (256, 256)])
+def test_paged_fp8_default_partitions(d, keys):
+    """Without split_len: the dense policy for rows of fewer than 256 bytes, the paged one at D=256."""
+    announce(f"paged fp8 default partitions d={d}")
+    b, hkv, n = 8, 32, 1000
+    q, (k8, ks, v8, vs), (kc, vc, ksp, vsp, bt, sl) = _fp8_dense_and_paged(b, hkv, hkv, 1, n, d, 64, torch.float16)
+    dense = fused_attn.attention_fp8(q, k8, ks, v8, vs, split_len=keys)
+    assert default_paged_split_len(1, n, b, hkv, 1, d) == keys
+    assert torch.equal(fused_attn.attention_paged(q, kc, vc, bt, sl, k_scale=ksp, v_scale=vsp), dense)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -141,7 +153,8 @@ def test_paged_fp8_decode_cache_bit_identical_to_dense():
     v8, vs = fused_attn.quantize_kv_fp8(randn(b, hkv, n, d, dtype=torch.bfloat16, gen=gen))
     kc, vc, ksp, vsp, bt, sl = fused_attn.paged_from_dense_fp8(k8, ks, v8, vs, 64,
                                                                generator=torch.Generator().manual_seed(7))
-    for split_len in (128, fused_attn.ops.default_split_len(1, n, b, hkv, hq // hkv)):
-        dense = fused_attn.attention_fp8(q, k8, ks, v8, vs, split_len=split_len)
+    for split_len in (128, None):
+        sk = split_len or default_paged_split_len(1, n, b, hkv, hq // hkv, d)
+        dense = fused_attn.attention_fp8(q, k8, ks, v8, vs, split_len=sk)
         paged = fused_attn.attention_paged(q, kc, vc, bt, sl, split_len=split_len, k_scale=ksp, v_scale=vsp)
         assert torch.equal(dense, paged), split_len
