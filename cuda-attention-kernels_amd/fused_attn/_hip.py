@@ -132,14 +132,22 @@ def library_path() -> str:
     return os.environ.get("FUSED_ATTN_HIP_LIB") or os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
 
 
+def _has_fwd_workspace(lib: ctypes.CDLL) -> bool:
+    return isinstance(getattr(lib, "fa_attention_fwd_ws", None), lib._FuncPtr)
+
+
 def _bind(lib: ctypes.CDLL) -> None:
     P = ctypes.POINTER(FwdParams)
     lib.fa_attention_fwd.argtypes = [P, ctypes.c_void_p]
     lib.fa_attention_fwd.restype = ctypes.c_int
-    lib.fa_attention_fwd_workspace_bytes.argtypes = [P]
-    lib.fa_attention_fwd_workspace_bytes.restype = ctypes.c_size_t
-    lib.fa_attention_fwd_ws.argtypes = [P, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
-    lib.fa_attention_fwd_ws.restype = ctypes.c_int
+    if _has_fwd_workspace(lib):
+        lib.fa_attention_fwd_workspace_bytes.argtypes = [P]
+        lib.fa_attention_fwd_workspace_bytes.restype = ctypes.c_size_t
+        lib.fa_attention_fwd_ws.argtypes = [P, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+        lib.fa_attention_fwd_ws.restype = ctypes.c_int
+    else:  # a library of this ABI from before the pair was added: no key splits
+        lib.fa_attention_fwd_workspace_bytes = lambda p: 0
+        lib.fa_attention_fwd_ws = lambda p, ws, nbytes, stream: lib.fa_attention_fwd(p, stream)
     lib.fa_attention_varlen_fwd.argtypes = [P, ctypes.c_void_p]
     lib.fa_attention_varlen_fwd.restype = ctypes.c_int
     lib.fa_splitk_workspace_bytes.argtypes = [ctypes.c_int32] * 5
@@ -159,8 +167,6 @@ def _bind(lib: ctypes.CDLL) -> None:
     lib.fa_device_supported.restype = ctypes.c_int32
     lib.fa_last_error.argtypes = []
     lib.fa_last_error.restype = ctypes.c_char_p
-    lib.fa_abi_version.argtypes = []
-    lib.fa_abi_version.restype = ctypes.c_int32
 
 
 def load_library() -> ctypes.CDLL:
@@ -177,14 +183,14 @@ def load_library() -> ctypes.CDLL:
             raise RuntimeError(f"fused_attn HIP backend unavailable: {_lib_error}")
         try:
             lib = ctypes.CDLL(path)
-            _bind(lib)
         except OSError as e:
             _lib_error = str(e)
             raise RuntimeError(f"fused_attn HIP backend unavailable: {e}") from e
-        got = lib.fa_abi_version()
+        got = lib.fa_abi_version()  # before the rest is bound, which another version need not have
         if got != ABI_VERSION:
             _lib_error = f"ABI version mismatch: library {got}, bindings {ABI_VERSION}"
             raise RuntimeError(f"fused_attn HIP backend unavailable: {_lib_error}")
+        _bind(lib)
         _lib = lib
         return lib
 
@@ -228,7 +234,7 @@ def _enable_native(index: int) -> None:
     """Let the native kernels serve device ``index``, which ``device_supported`` has accepted."""
     hip = load_library()
     with _lock:
-        if _native is not None:
+        if _native is not None and _has_fwd_workspace(hip):
             if not _native_devices:
                 _native.fa_torch_bind(*(ctypes.cast(f, ctypes.c_void_p) for f in (
                     hip.fa_attention_fwd_workspace_bytes, hip.fa_attention_fwd_ws, hip.fa_splitk_workspace_bytes,

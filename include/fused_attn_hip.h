@@ -28,6 +28,8 @@
 extern "C" {
 #endif
 
+/* Raised by changes that an older caller or library does not survive; added functions keep it
+   (fa_attention_fwd_ws and its size query came within 6: look them up before use). */
 #define FA_ABI_VERSION 6
 
 /* Element types (reference: DType, csrc/flash_attn.h:7). */

@@ -375,3 +375,35 @@ def test_views_with_token_strides_past_the_abi_bound_are_copied():
         out = _hip._aligned_view(view, 8, 16)
         assert out.data_ptr() != view.data_ptr() and out.is_contiguous() and torch.equal(out, view)
     assert _hip._aligned_view(below, 8, 16) is below
+
+
+def _other_library(tmp_path, monkeypatch, version, names):
+    """_hip with a library that exports fa_abi_version and, as functions that return 42, ``names``."""
+    import subprocess
+
+    src = tmp_path / "other.c"
+    src.write_text(f"int fa_abi_version(void) {{ return {version}; }}\n" + "".join(f"int {n}() {{ return 42; }}\n" for n in names))
+    subprocess.run(["cc", "-shared", "-fPIC", "-w", str(src), "-o", str(tmp_path / "other.so")], check=True)
+    monkeypatch.setenv("FUSED_ATTN_HIP_LIB", str(tmp_path / "other.so"))
+    monkeypatch.setattr(_hip, "_lib", None)
+    monkeypatch.setattr(_hip, "_lib_error", None)
+
+
+def test_library_without_key_splits_is_accepted(tmp_path, monkeypatch):
+    """A library of this ABI version from before fa_attention_fwd_ws was added: fa_attention_fwd serves its calls, and
+    the native dispatcher kernels, which call the pair, stay off."""
+    names = [n for n in _declared_functions() if not n.startswith("fa_attention_fwd_w") and n != "fa_abi_version"]
+    _other_library(tmp_path, monkeypatch, 6, names)
+    lib = _hip.load_library()
+    p = _params()
+    assert lib.fa_attention_fwd_workspace_bytes(p) == 0
+    assert lib.fa_attention_fwd_ws(p, None, 0, 0) == 42
+    monkeypatch.setattr(_hip, "_native", object())  # would raise on use
+    monkeypatch.setattr(_hip, "_native_devices", set())
+    _hip._enable_native(0)
+
+
+def test_library_of_another_version_is_named(tmp_path, monkeypatch):
+    _other_library(tmp_path, monkeypatch, 7, [])
+    with pytest.raises(RuntimeError, match="ABI version mismatch: library 7, bindings 6"):
+        _hip.load_library()
