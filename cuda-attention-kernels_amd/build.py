@@ -65,7 +65,9 @@ def _torch_commands() -> list[list[str]]:
     inc, lib = os.path.join(root, "include"), os.path.join(root, "lib")
     rocm = os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include")
     obj = os.path.join(BUILD_DIR, "fa_torch.o")
-    compile_ = [HIPCC, "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+    # the build that fused_attn/_hip.py asks for when it loads the library
+    build_ = f'-DFA_TORCH_BUILD="{torch.__version__} {torch.version.git_version}"'
+    compile_ = [HIPCC, "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM", build_,
                 f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-isystem", inc,
                 "-isystem", os.path.join(inc, "torch", "csrc", "api", "include"), "-isystem", rocm,
                 "-c", os.path.join(CSRC, TORCH_SOURCE), "-o", obj]

@@ -179,10 +179,25 @@ at::Tensor attention_autograd(c10::DispatchKeySet ks, const at::Tensor& q, const
 
 }  // namespace
 
-TORCH_LIBRARY_IMPL(fused_attn, CUDA, m) { m.impl("attention", TORCH_FN(attention_gpu)); }
-TORCH_LIBRARY_IMPL(fused_attn, AutogradCUDA, m) { m.impl("attention", TORCH_FN(attention_autograd)); }
-
 extern "C" {
+
+// What this library was built against: a torch build has no stable C++ ABI, and the HIP library bound below may come
+// from elsewhere.  Python compares them before it registers the kernels, so loading the library has no effect.
+const char* fa_torch_built_for(void) { return FA_TORCH_BUILD; }
+int32_t fa_torch_abi_version(void) { return FA_ABI_VERSION; }
+size_t fa_torch_params_size(void) { return sizeof(fa_fwd_params); }
+
+// Registers the kernels, once; 0 when torch refuses them.
+int32_t fa_torch_register(void) {
+  try {
+    static torch::Library cuda(torch::Library::IMPL, "fused_attn", c10::DispatchKey::CUDA, __FILE__, __LINE__);
+    static torch::Library autograd(torch::Library::IMPL, "fused_attn", c10::DispatchKey::AutogradCUDA, __FILE__, __LINE__);
+    static const bool once = (cuda.impl("attention", TORCH_FN(attention_gpu)), autograd.impl("attention", TORCH_FN(attention_autograd)), true);
+    return once;
+  } catch (const std::exception&) {
+    return 0;
+  }
+}
 
 void fa_torch_bind(void* fwd_workspace_bytes, void* fwd_ws, void* splitk_workspace_bytes, void* splitk, void* last_error) {
   g_abi.fwd_workspace_bytes = (decltype(g_abi.fwd_workspace_bytes))fwd_workspace_bytes;

@@ -209,16 +209,25 @@ _native_devices: set[int] = set()
 
 
 def load_native() -> None:
-    """Load the native dispatcher kernels of ``fused_attn::attention`` (csrc/fa_torch.cpp), if they are built for this
-    torch: they hand every call back to the Python kernels until ``_enable_native`` names its device."""
+    """Load and register the native dispatcher kernels of ``fused_attn::attention`` (csrc/fa_torch.cpp), if they are
+    built for this very torch (there is no stable C++ ABI: another build's symbols may resolve and still read its
+    tensors wrongly) and these bindings: they hand every call back to the Python kernels until ``_enable_native``
+    names its device."""
     global _native
     path = os.path.join(os.path.dirname(os.path.abspath(__file__)), TORCH_LIB_NAME)
     if _native is not None or torch.version.hip is None or not os.path.exists(path):
         return
+    want = (f"{torch.__version__} {torch.version.git_version}", ABI_VERSION, ctypes.sizeof(FwdParams))
     try:
-        torch.ops.load_library(path)
         lib = ctypes.CDLL(path)
-    except OSError as e:  # built for another torch
+        lib.fa_torch_built_for.restype = ctypes.c_char_p
+        lib.fa_torch_params_size.restype = ctypes.c_size_t
+        got = (lib.fa_torch_built_for().decode(), lib.fa_torch_abi_version(), lib.fa_torch_params_size())
+        if got != want:
+            raise OSError(f"built for torch, ABI version and parameter size {got}, found {want}")
+        if not lib.fa_torch_register():
+            raise OSError("torch refused its kernels")
+    except (OSError, AttributeError) as e:
         warnings.warn(f"fused_attn: {path} does not load, calls take the slower Python path: {e}")
         return
     lib.fa_torch_bind.argtypes = [ctypes.c_void_p] * 5

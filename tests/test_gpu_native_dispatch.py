@@ -25,6 +25,30 @@ def test_route_equals_the_python_rule():
         assert _hip._native.fa_torch_route(dtype != torch.float32, b, hkv * group, hkv, nq, nk, d) == want
 
 
+@pytest.mark.parametrize("name,value", [("fa_torch_built_for", '"2.9.9+rocm7.0 0123"'), ("fa_torch_abi_version", "5"),
+                                        ("fa_torch_params_size", "8"), ("fa_torch_register", "0"), (None, None)])
+def test_a_library_built_for_another_torch_is_not_registered(name, value, tmp_path, monkeypatch):
+    """A library that says it was built for another torch, ABI or parameter block (or one that says nothing: name None)
+    is left out with a warning, before it registers anything."""
+    import ctypes
+    import subprocess
+
+    has = {"fa_torch_built_for": f'"{torch.__version__} {torch.version.git_version}"', "fa_torch_abi_version": str(_hip.ABI_VERSION),
+           "fa_torch_params_size": str(ctypes.sizeof(_hip.FwdParams)), "fa_torch_register": "1"}
+    types = {"fa_torch_built_for": "const char*", "fa_torch_params_size": "unsigned long"}
+    lines = [] if name is None else [f"{types.get(n, 'int')} {n}(void) {{ {'registered++;' if n.endswith('register') else ''} return {value if n == name else v}; }}"
+                                     for n, v in has.items()]
+    (tmp_path / "other.c").write_text("int registered;\n" + "\n".join(lines))
+    subprocess.run(["cc", "-shared", "-fPIC", str(tmp_path / "other.c"), "-o", str(tmp_path / _hip.TORCH_LIB_NAME)], check=True)
+    monkeypatch.setattr(_hip, "__file__", str(tmp_path / "_hip.py"))
+    monkeypatch.setattr(_hip, "_native", None)
+    with pytest.warns(UserWarning, match="slower Python path"):
+        _hip.load_native()
+    assert _hip._native is None
+    registered = ctypes.c_int.in_dll(ctypes.CDLL(str(tmp_path / _hip.TORCH_LIB_NAME)), "registered").value
+    assert registered == (name == "fa_torch_register")
+
+
 @pytest.fixture
 def python_calls(monkeypatch):
     """Calls that reached the Python kernel, after one that let the device be found."""
