@@ -13,6 +13,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -63,13 +64,14 @@ def _torch_commands() -> list[list[str]]:
 
     root = os.path.dirname(os.path.abspath(torch.__file__))
     inc, lib = os.path.join(root, "include"), os.path.join(root, "lib")
+    python = sysconfig.get_paths()["include"]
     rocm = os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include")
     obj = os.path.join(BUILD_DIR, "fa_torch.o")
     # the build that fused_attn/_hip.py asks for when it loads the library
     build_ = f'-DFA_TORCH_BUILD="{torch.__version__} {torch.version.git_version}"'
     compile_ = [HIPCC, "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM", build_,
                 f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-isystem", inc,
-                "-isystem", os.path.join(inc, "torch", "csrc", "api", "include"), "-isystem", rocm,
+                "-isystem", os.path.join(inc, "torch", "csrc", "api", "include"), "-isystem", rocm, "-isystem", python,
                 "-c", os.path.join(CSRC, TORCH_SOURCE), "-o", obj]
     link = [HIPCC, "-shared", "-fPIC", obj, "-L", lib, "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-o",
             TORCH_OUT + ".tmp"]

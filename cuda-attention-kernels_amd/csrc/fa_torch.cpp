@@ -8,6 +8,8 @@
 //
 // The choice of kernel and partitions repeats ops._hip_kernel_for and ops.default_split_len
 // (fa_torch_route lets a test compare the two).
+#include <Python.h>
+
 #include <ATen/ATen.h>
 #include <ATen/core/dispatch/Dispatcher.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -82,6 +84,16 @@ int dtype_code(at::ScalarType t) {
   }
 }
 
+// Whether the environment names a backend.  Read with the GIL held (torch calls kernels without it): os.environ sets
+// variables under it, and a setenv beside this getenv may move the table it reads.
+bool backend_forced() {
+  const PyGILState_STATE gil = PyGILState_Ensure();
+  const char* forced = std::getenv("FUSED_ATTN_BACKEND");
+  const bool set = forced != nullptr && *forced != '\0';
+  PyGILState_Release(gil);
+  return set;
+}
+
 bool takes(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v) {
   if (q.dim() != 4 || k.dim() != 4 || v.dim() != 4 || !q.is_cuda() || !k.is_cuda() || !v.is_cuda()) return false;
   const int dev = q.device().index();
@@ -97,8 +109,7 @@ bool takes(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v) {
     }
   }
   if (!readable(q) || !readable(k) || !readable(v)) return false;
-  const char* forced = std::getenv("FUSED_ATTN_BACKEND");
-  return forced == nullptr || *forced == '\0';
+  return !backend_forced();
 }
 
 const c10::OperatorHandle& attention_op() {
@@ -211,6 +222,8 @@ void fa_torch_bind(void* fwd_workspace_bytes, void* fwd_ws, void* splitk_workspa
 void fa_torch_enable(int32_t index) {
   if (index >= 0 && index < 64) g_devices.fetch_or(uint64_t{1} << index, std::memory_order_release);
 }
+
+int32_t fa_torch_backend_forced(void) { return backend_forced(); }
 
 int64_t fa_torch_route(int32_t half, int64_t b, int64_t hq, int64_t hkv, int64_t nq, int64_t nk, int64_t d) {
   return route(half != 0, b, hq, hkv, nq, nk, d);

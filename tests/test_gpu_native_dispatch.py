@@ -1,5 +1,6 @@
 """The native dispatcher kernels of fused_attn::attention: same choice of kernel as the Python kernel, same results,
 and every call that they do not take reaches the Python kernel."""
+import os
 import random
 import threading
 
@@ -47,6 +48,35 @@ def test_a_library_built_for_another_torch_is_not_registered(name, value, tmp_pa
     assert _hip._native is None
     registered = ctypes.c_int.in_dll(ctypes.CDLL(str(tmp_path / _hip.TORCH_LIB_NAME)), "registered").value
     assert registered == (name == "fa_torch_register")
+
+
+def test_forced_backend_is_read_beside_threads_that_set_variables(monkeypatch):
+    """The environment is read under the GIL, as the Python kernel reads it: threads may assign variables meanwhile."""
+    forced = _hip._native.fa_torch_backend_forced  # (a ctypes call: without the GIL until the function takes it)
+    monkeypatch.delenv("FUSED_ATTN_BACKEND", raising=False)
+    assert not forced()
+    for value in ("splitk", "bogus"):
+        monkeypatch.setenv("FUSED_ATTN_BACKEND", value)
+        assert forced()
+    monkeypatch.setenv("FUSED_ATTN_BACKEND", "")
+    assert not forced()
+    stop = threading.Event()
+    names = [f"FUSED_ATTN_TEST_{i}" for i in range(500)]
+
+    def assign():
+        while not stop.is_set():
+            for n in names:  # growing the table moves it
+                os.environ[n] = "x" * 100
+            for n in names:
+                del os.environ[n]
+
+    thread = threading.Thread(target=assign)
+    thread.start()
+    try:
+        assert not any(forced() for _ in range(3000))
+    finally:
+        stop.set()
+        thread.join()
 
 
 @pytest.fixture
