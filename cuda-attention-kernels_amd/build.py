@@ -78,10 +78,17 @@ def _torch_commands() -> list[list[str]]:
     return [compile_, link]
 
 
+def _build_torch() -> None:
+    for cmd in _torch_commands():
+        _run(cmd)
+    os.replace(TORCH_OUT + ".tmp", TORCH_OUT)
+
+
 def build(verbose: bool = False) -> str:
+    """Build the libraries.  The dispatcher library is optional (without it calls take the Python path) and needs
+    torch's and Python's headers: where it does not build, that is said and the others are built all the same."""
     os.makedirs(BUILD_DIR, exist_ok=True)
-    torch_compile, torch_link = _torch_commands()
-    cmds = [torch_compile]
+    cmds = []
 
     def objects(sources):
         objs = []
@@ -92,18 +99,23 @@ def build(verbose: bool = False) -> str:
         return objs
 
     libs = [(LIB_OUT, objects(SOURCES)), (PROBE_OUT, objects(PROBE_SOURCES))]
-    with ThreadPoolExecutor(max_workers=len(cmds)) as ex:
+    with ThreadPoolExecutor(max_workers=len(cmds) + 1) as ex:
+        torch_lib = ex.submit(_build_torch)
         list(ex.map(_run, cmds))
-    _run(torch_link)
-    os.replace(TORCH_OUT + ".tmp", TORCH_OUT)
-    if verbose:
-        print(f"built {TORCH_OUT}")
-    for out, objs in libs:
-        tmp = out + ".tmp"
-        _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp])
-        os.replace(tmp, out)
-        if verbose:
-            print(f"built {out}")
+        for out, objs in libs:
+            tmp = out + ".tmp"
+            _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp])
+            os.replace(tmp, out)
+            if verbose:
+                print(f"built {out}")
+        try:
+            torch_lib.result()
+            if verbose:
+                print(f"built {TORCH_OUT}")
+        except Exception as e:
+            if os.path.exists(TORCH_OUT):  # an older one would not match the sources
+                os.remove(TORCH_OUT)
+            print(f"{TORCH_OUT} NOT built, attention() takes its slower Python path: {e}", file=sys.stderr)
     return LIB_OUT
 
 
