@@ -116,6 +116,7 @@ fa_status fa_attention_fwd(const fa_fwd_params* p, void* stream) {
 }
 
 size_t fa_attention_fwd_workspace_bytes(const fa_fwd_params* p) {
+  g_last_error.clear();
   if (validate(p, /*varlen=*/false, /*fp8_ok=*/false, /*generic_ok=*/true) != FA_OK) return 0;
   if (p->batch == 0 || p->seqlen_q == 0) return 0;
   return fa::fwd_workspace_bytes(*p);

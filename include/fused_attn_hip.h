@@ -103,7 +103,8 @@ typedef struct fa_fwd_params {
 fa_status fa_attention_fwd(const fa_fwd_params* p, void* stream);
 
 /* Bytes of workspace fa_attention_fwd_ws wants for these parameters: 0 for a grid that fills the GPU
-   by itself, else room for the fp32 partials of the key splits it is cut into (o, (max, sum)). */
+   by itself, else room for the fp32 partials of the key splits it is cut into (o, (max, sum)).
+   Also 0 for parameters that the call would refuse: fa_last_error() is then not empty. */
 size_t fa_attention_fwd_workspace_bytes(const fa_fwd_params* p);
 
 /* fa_attention_fwd with a caller workspace of at least fa_attention_fwd_workspace_bytes (16-byte

@@ -377,6 +377,44 @@ def test_views_with_token_strides_past_the_abi_bound_are_copied():
     assert _hip._aligned_view(below, 8, 16) is below
 
 
+def _dense(b, hq, hkv, nq, nk, d, causal=1, **over):
+    return _params(batch=b, heads_q=hq, heads_kv=hkv, seqlen_q=nq, seqlen_k=nk, head_dim=d, causal=causal,
+                   q_stride_b=hq * nq * d, q_stride_h=nq * d, q_stride_n=d, o_stride_b=hq * nq * d, o_stride_h=nq * d, o_stride_n=d,
+                   k_stride_b=hkv * nk * d, k_stride_h=nk * d, k_stride_n=d, v_stride_b=hkv * nk * d, v_stride_h=nk * d,
+                   v_stride_n=d, **over)
+
+
+@pytest.mark.parametrize("shape,splits", [((1, 4, 1, 70, 3000, 128), 8), ((1, 4, 1, 300, 4097, 128), 16), ((1, 3, 1, 64, 2500, 256), 16)])
+def test_fwd_workspace(lib, shape, splits):
+    """The size of a call that is cut up, and a workspace that does not hold it, refused before any launch."""
+    b, hq, _, nq, _, d = shape
+    p = _dense(*shape)
+    need = lib.fa_attention_fwd_workspace_bytes(p)
+    assert need == splits * b * hq * nq * (d + 2) * 4
+    for ws, size in ((None, need), (None, 0), (0x10000, need - 1), (0x10000, 0), (0x10004, need + 16)):
+        assert lib.fa_attention_fwd_ws(p, ws, size, None) == _hip.FA_ERR_WORKSPACE
+        assert "workspace" in lib.fa_last_error().decode()
+
+
+@pytest.mark.parametrize("p", [
+    _dense(8, 32, 8, 512, 4096, 128),  # fills the GPU
+    _dense(1, 4, 1, 70, 100, 128),  # few keys
+    _dense(1, 4, 1, 70, 3000, 128, dtype=_hip.F32, kv_dtype=_hip.F32),
+    _dense(0, 4, 1, 70, 3000, 128), _dense(1, 4, 1, 0, 3000, 128), _dense(1, 4, 1, 70, 0, 128),
+])
+def test_fwd_workspace_not_needed(lib, p):
+    assert lib.fa_attention_fwd_workspace_bytes(p) == 0 and lib.fa_last_error() == b""
+
+
+def test_fwd_workspace_of_a_refused_call(lib):
+    p = _dense(1, 4, 1, 70, 3000, 128, scale=float("nan"))
+    assert lib.fa_attention_fwd_workspace_bytes(p) == 0 and b"NaN" in lib.fa_last_error()
+    assert lib.fa_attention_fwd_ws(p, None, 0, None) == _hip.FA_ERR_INVALID_ARGUMENT
+    assert lib.fa_attention_fwd_workspace_bytes(None) == 0
+    good = _dense(1, 4, 1, 70, 3000, 128)
+    assert lib.fa_attention_fwd_workspace_bytes(good) > 0 and lib.fa_last_error() == b""
+
+
 def _other_library(tmp_path, monkeypatch, version, names):
     """_hip with a library that exports fa_abi_version and, as functions that return 42, ``names``."""
     import subprocess
