@@ -392,12 +392,13 @@ def bench_decode_sweep(steps, warmup):
         splits = fused_attn.choose_num_splits(c["b"], c["hq"], n, 1, cus)
         default = fused_attn.ops.default_split_len(1, n, c["b"], c["hkv"], c["hq"] // c["hkv"])
         variants = (
-            ("single_pass", "single-pass prefill kernel (no key split)",
+            # (the reference's single-pass row; attention_triton here cuts the keys of such a call over workgroups)
+            ("single_pass", "prefill kernel (attention_triton), its keys cut over workgroups where that pays",
              lambda: attention_triton(q, k, v, causal=True), kv16, (k, v)),
             ("splitk_ref_heuristic", f"split-K, {splits} splits (the reference's choose_num_splits over {cus} CUs)",
              lambda: fused_attn.attention_splitk(q, k, v, causal=True, num_splits=splits), kv16, (k, v)),
-            # called as the reference's benchmark calls its split-K function (bench_decode.py:53-54), not
-            # through the custom op, whose dispatch adds host time the other rows do not pay
+            # called as the reference's benchmark calls its split-K function (bench_decode.py:53-54); the custom
+            # op launches the same kernels from its native dispatcher kernel, with less host time
             ("splitk_default", f"split-K, {default}-key partitions (attention_splitk's default policy)",
              lambda: fused_attn.attention_splitk(q, k, v, causal=True), kv16, (k, v)),
             ("fp8_kv", "FP8-KV split-K (e4m3fn + fp32 per-64-key scales), default partitions",
