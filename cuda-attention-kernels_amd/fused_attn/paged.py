@@ -67,11 +67,12 @@ def default_paged_split_len(seqlen_q: int, max_seqlen_k: int, batch: int, heads_
     The grid is laid out for the longest sequence and the workgroups past a shorter one's end exit at
     once, so a ragged batch fills about half of it: it takes more, shorter partitions than a dense cache
     to keep the GPU busy to the end.  The longest power of two (other lengths measured up to 15% slower)
-    with 2304 workgroups at 256-byte rows (D=128 in 16 bits; half as many at twice the bytes), 512 to 4096; a
-    batch too small for that takes 128 or longer, with 1000 workgroups.
+    with 2048 workgroups at 256-byte rows (D=128 in 16 bits; 1152 at longer ones), 512 to 4096; a batch too
+    small for that takes 128 or longer, with 1000 workgroups.
     D=128 bf16 Hkv=8, ragged, us at this length and at the dense policy's: 48 sequences up to 8192 keys
     132 (1024) and 150 (1408); 100 up to 2000, 81 (512) and 87 (704); 16 up to 4096 with Hkv=4, 25 (256)
-    and 31 (128).
+    and 31 (128).  Half of a power of two that reaches the target is too short: 64 equal sequences of 4096
+    keys 170 (1024) and 184 (512), 32 of 16384 with Hkv=4 and 4 queries 197 (1024) and 217 (512).
 
     Rows of fewer than 256 bytes (D=64, FP8 at D=64 and D=128) take the dense policy: a short partition is
     then half a partial's traffic, and what shorter ones gain for some ragged batches they lose for others
@@ -83,7 +84,7 @@ def default_paged_split_len(seqlen_q: int, max_seqlen_k: int, batch: int, heads_
     rows = group * seqlen_q
     items = max(1, batch * heads_kv * -(-rows // 128))
     keys = 4096
-    while keys > 512 and items * -(-max_seqlen_k // keys) < 2304 * 256 / row_bytes:
+    while keys > 512 and items * -(-max_seqlen_k // keys) < (2048 if row_bytes == 256 else 1152):
         keys //= 2
     while keys > 128 and items * -(-max_seqlen_k // keys) < 1000:
         keys //= 2

@@ -63,10 +63,10 @@ def test_fp8_two_partitions_per_workgroup():
 @pytest.mark.parametrize("n", [0, 1, 600, 8192, 1 << 20])
 @pytest.mark.parametrize("b,hkv,group,nq", [(1, 1, 1, 1), (16, 4, 4, 1), (48, 8, 4, 1), (100, 8, 4, 4), (300, 32, 8, 16)])
 def test_default_partitions(b, hkv, group, nq, n, row_bytes):
-    """The longest power of two whose grid reaches its target: 2304 workgroups (by 256-byte rows) down to 512 keys,
-    1000 below."""
+    """The longest power of two whose grid reaches its target: 2048 workgroups (1152 above 256-byte rows) down to 512
+    keys, 1000 below."""
     keys = default_paged_split_len(nq, n, b, hkv, group, row_bytes)
-    large = 2304 * 256 // row_bytes
+    large = 2048 if row_bytes == 256 else 1152
 
     def workgroups(length):
         return b * hkv * -(-group * nq // 128) * -(-n // length)
@@ -79,6 +79,7 @@ def test_default_partitions(b, hkv, group, nq, n, row_bytes):
 @pytest.mark.parametrize("args,keys", [
     ((1, 8192, 48, 8, 4, 256), 1024), ((1, 2000, 100, 8, 4, 256), 512), ((1, 4096, 16, 4, 4, 256), 256),
     ((1, 2000, 100, 8, 4, 512), 1024),
+    ((1, 4096, 64, 8, 4, 256), 1024), ((4, 16384, 32, 4, 8, 256), 1024), ((1, 32768, 32, 8, 4, 256), 4096),
     # rows of fewer than 256 bytes: the dense policy
     ((8, 8192, 48, 8, 4, 128), 1408), ((16, 4000, 24, 8, 8, 64), 384), ((1, 3000, 4, 32, 4, 128), 192),
 ])
