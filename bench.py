@@ -367,7 +367,7 @@ PREFILL_SWEEP = dict(b=2, hq=32, hkv=8, d=128, n=(2048, 8192, 16384))
 def bench_decode_sweep(steps, warmup):
     """Single-sequence decode across context lengths (the reference's decode benchmark,
     benchmarks/bench_decode.py:30-65: batch 1, Hq=32, Hkv=8, D=128, one fp16 query, causal, contexts
-    4096/16384/65536): the single-pass prefill kernel, split-K with the reference's split heuristic
+    4096/16384/65536): the prefill kernel (which cuts the keys), split-K with the reference's split heuristic
     (choose_num_splits over the GPU's 256 CUs), split-K with attention_splitk's default partitions, and
     the FP8 KV cache at its default partitions.  GB/s counts each variant's own K/V (+ scale) bytes."""
     import torch

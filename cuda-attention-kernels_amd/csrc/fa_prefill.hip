@@ -723,7 +723,7 @@ FwdPlan plan_fwd(const fa_fwd_params& p, bool varlen, bool workspace) {
   // cuts each block's keys over several workgroups.  The estimate below, in microseconds, charges
   // a CU 1.0 per 128-query tile it runs with two waves per SIMD, 1.15 with one, 0.8 at D=256 (whose
   // workgroups run one per CU); the partials 0.4 per MB (written and read back) and the second
-  // launch 10 (4 on the GPU, the rest on the host).  512 queries against 16384 keys (Hq=32 Hkv=8
+  // launch 10 (4 on the GPU, the rest on the host where Python launches it; the op's native kernel needs about 2).  512 queries against 16384 keys (Hq=32 Hkv=8
   // D=128 causal, 128 row blocks): 223 us unsplit, 132 with 4 splits of 256-query blocks (8
   // splits: 143 with 128-query blocks); 64 queries against 33000: 441 -> 68; 1000 queries against
   // 3000 (256 row blocks) stay unsplit at 52 (2 splits: 58).
