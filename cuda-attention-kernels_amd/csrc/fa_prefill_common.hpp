@@ -61,9 +61,11 @@ inline int prefill_share(bool causal, int64_t heads) { return causal && heads % 
 // Heads that do not divide are dealt to the XCDs rank by rank where that beats one order over all heads: grids
 // of more than one workgroup per CU, with fewer than 32 heads or D <= 64 (D=64 B=7 Hq=12 N=1500 49.1 -> 38.6
 // us; 25 heads N=1300 D=128 35.5 -> 27.5).  Dealt, every XCD reads every K/V: with more heads at D >= 128 that
-// can cost what the balance gains (B=9 Hq=12 Hkv=4 N=1500, D=128 94.8 -> 86.6, D=256 176 -> 187).
-inline bool prefill_deal(bool causal, int64_t heads, int64_t total, int head_dim) {
-  return causal && heads % 8 != 0 && total > 256 && (heads < 32 || head_dim <= 64);
+// can cost what the balance gains (B=9 Hq=12 Hkv=4 N=1500, D=128 94.8 -> 86.6, D=256 176 -> 187), and so it
+// does where the first row block sees more than half of what the last one sees (D=64 B=7 Hq=20, 178 queries on
+// 565 keys 18.0 -> 19.7).
+inline bool prefill_deal(bool causal, int64_t heads, int64_t total, int head_dim, int nq, int nk) {
+  return causal && heads % 8 != 0 && total > 256 && (heads < 32 || head_dim <= 64) && 2 * ((int64_t)nk - nq + 128) <= nk;
 }
 inline int64_t prefill_units(bool causal, int64_t heads, int group, int nk, int head_dim) {
   const int64_t most = std::min<int64_t>(prefill_unit_heads(nk, head_dim, group), heads);
@@ -74,12 +76,12 @@ inline int64_t prefill_units(bool causal, int64_t heads, int group, int nk, int 
   return (even + group - 1) / group * group;  // whole kv-heads: at most `most`, itself a multiple of group
 }
 
-// The schedule fields of a dense call's arguments (kv_groups, group, nk, causal, n_rowblk and total are set;
+// The schedule fields of a dense call's arguments (kv_groups, group, nq, nk, causal, n_rowblk and total are set;
 // nw: waves per workgroup).
 inline void prefill_schedule(TileArgs& a, int head_dim, int nw) {
   const bool causal = a.causal != 0;
   const int64_t heads = (int64_t)a.kv_groups * a.group;
-  a.deal = prefill_deal(causal, heads, a.total, head_dim);
+  a.deal = prefill_deal(causal, heads, a.total, head_dim, a.nq, a.nk);
   a.share = prefill_share(causal, heads);
   // at most `heads`, so that u_items <= total
   a.u_heads = (int32_t)(a.deal ? heads : prefill_units(causal, heads, a.group, a.nk, head_dim));

@@ -13,16 +13,18 @@ CSRC = os.path.join(ROOT, "cuda-attention-kernels_amd", "csrc")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 SOURCE = """
 #include "fa_prefill_common.hpp"
-extern "C" void schedule(int heads_kv, int group, int nk, int head_dim, int n_rowblk, int causal, int nw, int* out) {
+extern "C" void schedule(int heads_kv, int group, int nq, int nk, int head_dim, int n_rowblk, int causal, int nw, int* out) {
   fa::TileArgs a{};
   a.kv_groups = heads_kv;
   a.group = group;
+  a.nq = nq;
   a.nk = nk;
   a.causal = causal;
   a.n_rowblk = n_rowblk;
   a.total = heads_kv * group * n_rowblk;
   fa::prefill_schedule(a, head_dim, nw);
   *out++ = a.u_heads;
+  *out++ = a.deal;
   for (int i = 0; i < a.total; ++i) {
     const fa::PrefillOrder o = fa::prefill_dense_order(a, (uint32_t)i);
     *out++ = (int)o.head;
@@ -41,13 +43,14 @@ def schedule(tmp_path_factory):
                     "-o", str(lib)], check=True, capture_output=True)
     c = ctypes.CDLL(str(lib)).schedule
 
-    def run(heads_kv, group, n, d, causal, nw=4):
+    def run(heads_kv, group, n, d, causal, nw=4, nk=None):
         n_rowblk = -(-n // (32 * nw))
         total = heads_kv * group * n_rowblk
-        out = (ctypes.c_int * (1 + 2 * total))()
-        c(heads_kv, group, n, d, n_rowblk, int(causal), nw, out)
-        items = list(zip(out[1::2], out[2::2]))
+        out = (ctypes.c_int * (2 + 2 * total))()
+        c(heads_kv, group, n, nk or n, d, n_rowblk, int(causal), nw, out)
+        items = list(zip(out[2::2], out[3::2]))
         assert sorted(items) == [(h, r) for h in range(heads_kv * group) for r in range(n_rowblk)]
+        run.dealt = bool(out[1])
         return items, out[0], n_rowblk
 
     return run
@@ -79,3 +82,14 @@ def test_xcds_share_causal_work_evenly(schedule, b, hkv, group, n):
         assert x[0][1] == 0 and x[-1][1] == n_rowblk - 1  # from a heaviest to a lightest block
         # within a unit the ranks go down; a unit starts over at most once every `unit` heads
         assert sum(p[1] > q[1] for p, q in zip(x, x[1:])) == -(-(b * hkv * group // 8) // unit) - 1
+
+
+@pytest.mark.parametrize("heads_kv,group,nq,nk,d,dealt", [
+    (28, 1, 1300, 1300, 128, True), (84, 1, 1500, 1500, 64, True), (108, 1, 1500, 1500, 128, False),
+    (35, 4, 178, 565, 64, False), (35, 4, 565, 565, 64, True),  # the first row block sees most of the keys, or few
+    (20, 1, 500, 500, 128, False),  # one workgroup per CU
+    (32, 1, 1300, 1300, 128, False),  # the heads divide
+])
+def test_which_calls_are_dealt(schedule, heads_kv, group, nq, nk, d, dealt):
+    schedule(heads_kv, group, nq, d, True, 4, nk)
+    assert schedule.dealt == dealt
