@@ -30,6 +30,7 @@
 #include <float.h>
 
 #include <algorithm>
+#include <cmath>
 
 #include <type_traits>
 
@@ -374,8 +375,10 @@ hipError_t launch_f32(const TileArgs& a, bool key_split, hipStream_t stream) {
 // Both in units of one 32-key tile of a 4-wave workgroup, per compute unit: the plain kernel takes its
 // heaviest row block or the mean load of the 256 CUs, whichever is longer; KS takes a quarter of the tiles, 10%
 // more for K/V that four times as many workgroups fetch, and 1.1 tiles to start and merge each workgroup.
-// D=64, causal unless said, us plain and KS: B=2 H=4 N=256 22.3 and 10.0; 8 heads N=1000 74.9 and 25.2; B=4 H=8
-// N=1000 78.2 and 59.6 (not causal 84.4 and 95.9); B=8 H=16 N=256 24.6 and 29.4; B=8 H=16 N=2048 570 and 725.
+// At D=128 a CU runs one KS workgroup with a single stage, so a started round counts whole (not causal, B=11 H=8
+// N=151, 440 workgroups: 31.8 and 36.6).  D=64, causal unless said, us plain and KS: B=2 H=4 N=256 22.3 and 10.0; 8
+// heads N=1000 74.9 and 25.2; B=4 H=8 N=1000 78.2 and 59.6 (not causal 84.4 and 95.9); B=8 H=16 N=256 24.6 and 29.4;
+// B=8 H=16 N=2048 570 and 725.
 static bool f32_key_split_pays(const fa_fwd_params& p) {
   constexpr double kCus = 256;
   const double heads = (double)p.batch * p.heads_q, tiles = (p.seqlen_k + 31) / 32;
@@ -385,7 +388,8 @@ static bool f32_key_split_pays(const fa_fwd_params& p) {
   };
   const double plain_wgs = heads * ((p.seqlen_q + 127) / 128), ks_wgs = heads * ((p.seqlen_q + 31) / 32);
   const double plain = std::max(tiles, plain_wgs * mean_tiles(128) / kCus);
-  const double ks = std::max(1.1 * tiles / 4 + 1.1, ks_wgs / kCus * (1.1 * (mean_tiles(32) + 1.5) / 4 + 1.1));
+  const double rounds = p.head_dim == 128 && ks_wgs > kCus ? std::ceil(ks_wgs / kCus) : ks_wgs / kCus;
+  const double ks = std::max(1.1 * tiles / 4 + 1.1, rounds * (1.1 * (mean_tiles(32) + 1.5) / 4 + 1.1));
   return ks < plain;
 }
 
